@@ -213,6 +213,7 @@ def _forward(ops, st):
     if family == "base_block":
         bank = torch.stack(st["queries"])
         inter, lse = ops.attention_residual_phase1(st["values"], bank, True)
+        inter, lse = inter.unbind(0), lse.unbind(0)
         reads = [inter[0]]
         for q in range(1, c["Q"]):
             reads.append(ops.attention_residual_phase2(

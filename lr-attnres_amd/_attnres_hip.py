@@ -266,6 +266,17 @@ def load() -> ctypes.CDLL:
     lib.attnres_keyed_logits_backward.restype = c_int
     lib.attnres_keyed_logits_backward.argtypes = [POINTER(KeyedLogitsDesc), c_void_p, POINTER(c_float),
                                                   POINTER(c_void_p), c_void_p, c_void_p, c_size_t, c_void_p]
+    lib.attnres_phase1_bank_fits.restype = c_int
+    lib.attnres_phase1_bank_fits.argtypes = [POINTER(KeyedLogitsDesc)]
+    lib.attnres_phase1_bank_forward.restype = c_int
+    lib.attnres_phase1_bank_forward.argtypes = [POINTER(KeyedLogitsDesc), c_void_p, POINTER(c_float), c_void_p,
+                                                POINTER(c_float), c_void_p]
+    lib.attnres_phase1_bank_backward_workspace_size.restype = c_size_t
+    lib.attnres_phase1_bank_backward_workspace_size.argtypes = [POINTER(KeyedLogitsDesc)]
+    lib.attnres_phase1_bank_backward.restype = c_int
+    lib.attnres_phase1_bank_backward.argtypes = [POINTER(KeyedLogitsDesc), c_void_p, POINTER(c_float), c_void_p,
+                                                 POINTER(c_float), POINTER(c_void_p), c_void_p, c_void_p, c_size_t,
+                                                 c_void_p]
     lib.attnres_phase2_forward.restype = c_int
     lib.attnres_phase2_forward.argtypes = [POINTER(Phase2Desc), c_void_p, c_void_p]
     lib.attnres_phase2_backward.restype = c_int
@@ -696,6 +707,42 @@ def keyed_logits_backward(desc: KeyedLogits, device, dtype, dlogits, inv_rms, wa
                                            dv_arr, _ptr(dq) if want_dq else None, _ptr(ws) if want_dq else None,
                                            ws_bytes, _stream(device))
     _check(rc, "keyed-logits backward")
+    return dvals, dq
+
+
+def phase1_bank_fits(desc: KeyedLogits) -> bool:
+    """Whether the one-pass query-bank kernels take this description (include/attnres_phase1_bank.h)."""
+    return bool(load().attnres_phase1_bank_fits(ctypes.byref(desc.c)))
+
+
+def phase1_bank_forward(desc: KeyedLogits, device, dtype, for_backward: bool):
+    """Returns (out [Q, n_tok, D], lse [Q, n_tok], logits [Q, S, n_tok] | empty, inv_rms [S, n_tok] | empty)."""
+    Q, n, S = desc.n_q, desc.n_tok, desc.n_src
+    out = torch.empty((Q, n, desc.D), device=device, dtype=dtype)
+    lse = torch.empty((Q, n), device=device, dtype=torch.float32)
+    logits = torch.empty((Q, S, n) if for_backward else (0,), device=device, dtype=dtype)
+    keep = bool(desc.c.key_norm) and for_backward
+    inv = torch.empty((S, n) if keep else (0,), device=device, dtype=torch.float32)
+    rc = load().attnres_phase1_bank_forward(ctypes.byref(desc.c), _ptr(out), _fptr(lse),
+                                            _ptr(logits) if for_backward else None, _fptr(inv) if keep else None,
+                                            _stream(device))
+    _check(rc, "query-bank forward")
+    return out, lse, logits, inv
+
+
+def phase1_bank_backward(desc: KeyedLogits, device, dtype, grad_out, grad_lse, logits, inv_rms, want_dq: bool):
+    """Returns (dvalues list of [n_tok, D], dqueries [Q, D] | None)."""
+    lib = load()
+    n = desc.n_src
+    dvals = _row_blocks(n, desc.n_tok, desc.D, device, dtype, True)
+    dv_arr = (c_void_p * n)(*[t.data_ptr() for t in dvals])
+    dq = torch.empty((desc.n_q, desc.D), device=device, dtype=dtype) if want_dq else None
+    ws_bytes = lib.attnres_phase1_bank_backward_workspace_size(ctypes.byref(desc.c)) if want_dq else 0
+    ws = torch.empty((max(1, ws_bytes),), device=device, dtype=torch.uint8) if want_dq else None
+    rc = lib.attnres_phase1_bank_backward(ctypes.byref(desc.c), _ptr(grad_out), _fptr(grad_lse), _ptr(logits),
+                                          _fptr(inv_rms) if inv_rms.numel() else None, dv_arr, _ptr(dq), _ptr(ws),
+                                          ws_bytes, _stream(device))
+    _check(rc, "query-bank backward")
     return dvals, dq
 
 

@@ -912,13 +912,50 @@ class _KeyedLogitsFn(torch.autograd.Function):
         return (None, dq, *[d if want[2 + i] else None for i, d in enumerate(dvals)])
 
 
+class _Phase1BankFn(torch.autograd.Function):
+    """Eager autograd of phase 1 from a query bank in one pass: inputs
+    (key_norm, queries [Q,D], *value rows); outputs (out [Q,n,D], lse [Q,n])."""
+
+    @staticmethod
+    def forward(ctx, key_norm, queries, *values):
+        ctx.set_materialize_grads(False)
+        v0 = values[0]
+        desc = _hip.KeyedLogits(values, queries, key_norm)
+        need = any(ctx.needs_input_grad)
+        with _device_ctx(v0.device):
+            out, lse, logits, inv = _hip.phase1_bank_forward(desc, v0.device, v0.dtype, need)
+        ctx.key_norm = key_norm
+        ctx.save_for_backward(queries, logits, inv, *values)
+        return out, lse
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, grad_out, grad_lse):
+        queries, logits, inv, *values = ctx.saved_tensors
+        if grad_out is None and grad_lse is None:
+            return (None, None, *([None] * len(values)))
+        v0 = values[0]
+        Q, n, D = queries.size(0), v0.size(0), v0.size(1)
+        grad_out = v0.new_zeros((Q, n, D)) if grad_out is None else grad_out.contiguous()
+        if grad_out.data_ptr() % 16:  # (a view into a larger gradient)
+            grad_out = grad_out.clone()
+        grad_lse = grad_lse.float().contiguous() if grad_lse is not None else None
+        want = ctx.needs_input_grad
+        with _device_ctx(v0.device):
+            dvals, dq = _hip.phase1_bank_backward(_hip.KeyedLogits(values, queries, ctx.key_norm), v0.device, v0.dtype,
+                                                  grad_out, grad_lse, logits, inv, bool(want[1]))
+        return (None, dq, *[d if want[2 + i] else None for i, d in enumerate(dvals)])
+
+
 def attention_residual_phase1(values, queries: Tensor, key_norm: bool, force_triton: bool = False):
     """Phase 1 with logits from a query bank (reference: attnres_ops.py:3862-3907; eager form
     ``_attnres_phase1_read_torch`` :2620-2627).
 
     values: S x [B,T,D] (list or stacked [S,B,T,D]); queries [Q,D], cast to the
-    value dtype as the reference does.  The logits ``<queries[q], rms_norm(v_s)>``
-    (value dtype) come from the keyed-logits kernels; the read over them is
+    value dtype as the reference does.  One pass each way scores the bank and
+    reads (up to 12 sources and sites, D a multiple of 4 up to 2048); other
+    shapes take the logits ``<queries[q], rms_norm(v_s)>`` (value dtype) from the
+    keyed-logits kernels and read over them with
     ``attention_residual_phase1_from_logits``.  Returns (out [Q,B,T,D], lse [Q,B,T]).
     """
     srcs = _sources(values)
@@ -937,6 +974,9 @@ def attention_residual_phase1(values, queries: Tensor, key_norm: bool, force_tri
     _check_gpu(srcs + [queries], "attention_residual_phase1")
     q = queries.to(srcs[0].dtype).contiguous()
     rows = [_rows2d(t) for t in srcs]
+    if not _compiling() and _hip.phase1_bank_fits(_hip.KeyedLogits(rows, q, key_norm)):
+        out, lse = _Phase1BankFn.apply(bool(key_norm), q, *rows)
+        return out.view(Q, B, T, D), lse.view(Q, B, T)
     logits = _KeyedLogitsFn.apply(bool(key_norm), q, *rows)
     return attention_residual_phase1_from_logits(srcs, logits.view(Q, len(srcs), B, T))
 

@@ -9,6 +9,7 @@
 #include <mutex>
 #include <string>
 
+#include "../../include/attnres_phase1_bank.h"
 #include "attnres_launch.h"
 #include "attnres_params.h"
 
@@ -1612,6 +1613,135 @@ void fill_keyed_logits(const attnres_keyed_logits_desc* d, KeyedLogitsParams* p,
 int64_t keyed_logits_groups(int64_t n_tok) { return n_tok < kKeyedLogitsGroups ? n_tok : kKeyedLogitsGroups; }
 
 }  // namespace
+
+// ---------------------------------------------------------------- phase 1 from a query bank, one pass
+namespace {
+
+// Shapes of attnres_phase1_bank.hip: a wave per 256 columns with four elements
+// per lane, at most eight waves, 12 source and 12 site slots (the register
+// budget: 12 sources and 12 sites take 228 VGPRs in the backward).
+bool phase1_bank_plan(const attnres_keyed_logits_desc* d, Phase1BankParams* p, Launch* L) {
+  if (d->n_tok <= 0 || d->n_src > kBankMaxSources || d->n_q > kBankMaxSites || d->dim > kBankMaxDim) return false;
+  if (d->dim % 4) return false;
+  const size_t row = 4 * elem_size(d->dtype);  // bytes of a lane's vector
+  if ((uintptr_t)d->queries % row) return false;
+  memset(p, 0, sizeof(*p));
+  for (int s = 0; s < d->n_src; ++s) {
+    if ((uintptr_t)d->values[s] % row || (size_t)d->value_row_stride[s] % 4) return false;
+    p->val[s] = d->values[s];
+    p->vstride[s] = (int32_t)d->value_row_stride[s];
+  }
+  p->queries = d->queries;
+  p->n_tok = d->n_tok;
+  p->n_src = d->n_src;
+  p->n_q = d->n_q;
+  p->D = d->dim;
+  p->key_norm = d->key_norm ? 1 : 0;
+  p->eps = d->norm_eps;
+  memset(L, 0, sizeof(*L));
+  L->wpt = (d->dim + 255) / 256;
+  auto slots = [](int n) { return n <= 8 ? (n + 1) / 2 * 2 : 12; };
+  L->nmax = slots(d->n_src);
+  L->teams = slots(d->n_q);
+  p->np = 2;
+  while (p->np < L->nmax) p->np <<= 1;
+  return true;
+}
+
+// Workgroups: each loads the bank once and walks tokens.  Backward workgroups
+// also write one partial row of Q * D sums; one resident round of three waves
+// per SIMD is best (attnres_phase1_bank.hip).  Forward, 2048 / 4096 / 16384:
+// 78 / 65 / 66 us at 6 sources, 4 sites, D = 768, 16384 tokens.
+constexpr int kBankFwdGroups = 4096;
+constexpr int kBankBwdGroups = 1280;
+int64_t bank_groups(int64_t n_tok, int64_t cap) { return n_tok < cap ? n_tok : cap; }
+
+}  // namespace
+
+extern "C" int attnres_phase1_bank_fits(const attnres_keyed_logits_desc* d) {
+  if (check_keyed_logits(d) != ATTNRES_OK) return 0;
+  Phase1BankParams p;
+  Launch L;
+  return phase1_bank_plan(d, &p, &L) ? 1 : 0;
+}
+
+extern "C" int attnres_phase1_bank_forward(const attnres_keyed_logits_desc* d, void* out, float* lse, void* logits,
+                                           float* inv_rms, void* stream) {
+  int rc = check_keyed_logits(d);
+  if (rc) return rc;
+  if (d->n_tok == 0) return ATTNRES_OK;
+  if (!out || !lse) return fail(ATTNRES_EINVAL, "out / lse is NULL");
+  Phase1BankParams p;
+  Launch L;
+  if (!phase1_bank_plan(d, &p, &L) || (uintptr_t)out % (4 * elem_size(d->dtype)))
+    return fail(ATTNRES_EUNSUPPORTED, "shape or alignment outside the one-pass query-bank kernels");
+  p.out = out;
+  p.lse = lse;
+  p.logits = logits;
+  p.inv = d->key_norm ? inv_rms : nullptr;
+  L.grid = (int)bank_groups(d->n_tok, kBankFwdGroups);
+  hipError_t err = launch_phase1_bank_forward(d->dtype, p, L, (hipStream_t)stream);
+  if (err != hipSuccess) return fail(ATTNRES_ELAUNCH, "query-bank forward launch failed: %s", hipGetErrorString(err));
+  return ATTNRES_OK;
+}
+
+extern "C" size_t attnres_phase1_bank_backward_workspace_size(const attnres_keyed_logits_desc* d) {
+  if (check_keyed_logits(d) != ATTNRES_OK || d->n_tok == 0) return 0;
+  return (size_t)bank_groups(d->n_tok, kBankBwdGroups) * part_stride(d->n_q * d->dim) * sizeof(float);
+}
+
+extern "C" int attnres_phase1_bank_backward(const attnres_keyed_logits_desc* d, const void* grad_out,
+                                            const float* grad_lse, const void* logits, const float* inv_rms,
+                                            void* const* dvalues, void* dqueries, void* workspace,
+                                            size_t workspace_bytes, void* stream) {
+  int rc = check_keyed_logits(d);
+  if (rc) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  if (d->n_tok == 0) {
+    if (dqueries) zero_async(dqueries, (size_t)d->n_q * d->dim * elem_size(d->dtype), st);
+    return ATTNRES_OK;
+  }
+  if (!grad_out || !logits || !dvalues) return fail(ATTNRES_EINVAL, "grad_out / logits / dvalues is NULL");
+  if (d->key_norm && !inv_rms) return fail(ATTNRES_EINVAL, "key_norm backward needs the forward's inv_rms");
+  const size_t row = 4 * elem_size(d->dtype);
+  Phase1BankParams p;
+  Launch L;
+  bool ok = phase1_bank_plan(d, &p, &L) && (uintptr_t)grad_out % row == 0;
+  for (int s = 0; ok && s < d->n_src; ++s) {
+    if (!dvalues[s]) return fail(ATTNRES_EINVAL, "dvalues[%d] is NULL", s);
+    ok = (uintptr_t)dvalues[s] % row == 0;
+    p.dval[s] = dvalues[s];
+  }
+  if (!ok) return fail(ATTNRES_EUNSUPPORTED, "shape or alignment outside the one-pass query-bank kernels");
+  p.gout = grad_out;
+  p.glse = grad_lse;
+  p.logits = const_cast<void*>(logits);
+  p.inv = const_cast<float*>(inv_rms);
+  L.grid = (int)bank_groups(d->n_tok, kBankBwdGroups);
+  if (dqueries) {
+    const size_t need = attnres_phase1_bank_backward_workspace_size(d);
+    if (!workspace || workspace_bytes < need)
+      return fail(ATTNRES_EWORKSPACE, "workspace of %zu bytes needed, got %zu", need,
+                  workspace ? workspace_bytes : (size_t)0);
+    p.partials = (float*)workspace;
+  }
+  hipError_t err = launch_phase1_bank_backward(d->dtype, p, L, st);
+  if (err != hipSuccess) return fail(ATTNRES_ELAUNCH, "query-bank backward launch failed: %s", hipGetErrorString(err));
+  if (dqueries) {
+    ReduceParams rp;
+    memset(&rp, 0, sizeof(rp));
+    rp.partials = p.partials;
+    rp.n_groups = L.grid;
+    rp.n_part = d->n_q * d->dim;
+    rp.layout = kPartTiled;
+    rp.n_q = rp.n_part;
+    rp.part_gate = rp.part_bias = rp.part_extra = -1;
+    rp.dquery = dqueries;
+    err = launch_reduce_partials(d->dtype, rp, st);
+    if (err != hipSuccess) return fail(ATTNRES_ELAUNCH, "reduce launch failed: %s", hipGetErrorString(err));
+  }
+  return ATTNRES_OK;
+}
 
 namespace {
 

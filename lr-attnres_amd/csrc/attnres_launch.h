@@ -61,6 +61,10 @@ hipError_t launch_phase2_fast_backward(int dtype, const Phase2Params& p, const L
 // kKLMaxQ floats; backward L.teams = query-gradient groups
 hipError_t launch_keyed_logits_forward(int dtype, const KeyedLogitsParams& p, const Launch& L, hipStream_t st);
 hipError_t launch_keyed_logits_backward(int dtype, const KeyedLogitsParams& p, const Launch& L, hipStream_t st);
+// phase 1 from a query bank in one pass: one workgroup of L.wpt = ceil(D / 256)
+// waves per token, L.nmax = source slots (2/4/6/8/12), L.teams = site slots (the same)
+hipError_t launch_phase1_bank_forward(int dtype, const Phase1BankParams& p, const Launch& L, hipStream_t st);
+hipError_t launch_phase1_bank_backward(int dtype, const Phase1BankParams& p, const Launch& L, hipStream_t st);
 // key-producer epilogue: one wave per token, L.teams waves per workgroup,
 // L.vec = 16-byte vectors for the output columns
 hipError_t launch_keyed_split_forward(int dtype, const KeySplitParams& p, const Launch& L, hipStream_t st);

@@ -294,6 +294,27 @@ struct Phase2Params {
   void* acc_dpk_old;           // [n_tok, R] or null
 };
 
+// Phase 1 from a query bank in one pass (attnres_phase1_bank.hip): rows of up
+// to 2048 elements, 12 sources and 12 sites
+constexpr int kBankMaxSources = 12, kBankMaxSites = 12, kBankMaxDim = 2048;
+struct Phase1BankParams {
+  const void* val[kBankMaxSources];
+  void* dval[kBankMaxSources];   // backward: [n_tok, D] dense
+  int32_t vstride[kBankMaxSources];
+  const void* queries;           // [Q, D] dense, value dtype
+  void* out;                     // forward: [Q, n_tok, D]
+  float* lse;                    // forward: [Q, n_tok]
+  void* logits;                  // [Q, S, n_tok], value dtype (forward writes unless null, backward reads)
+  float* inv;                    // [S, n_tok]: 1/rms of each key (key_norm; as logits)
+  const void* gout;              // backward: [Q, n_tok, D] dense
+  const float* glse;             // backward: [Q, n_tok] or null
+  float* partials;               // backward: bank-gradient partial sums, kPartTiled (null: none)
+  int64_t n_tok;
+  int32_t n_src, n_q, D, key_norm;
+  int32_t np;                    // lanes per softmax row: power of two >= the source slots
+  float eps;
+};
+
 // Logits of a query bank against the sources' keys (phase 1 from a query bank)
 constexpr int kKLMaxQ = 16;
 struct KeyedLogitsParams {

@@ -11,6 +11,7 @@
 
 #include "../../include/attnres_phase1_bank.h"
 #include "attnres_launch.h"
+#include "attnres_lr_split.h"
 #include "attnres_params.h"
 
 using namespace attnres;
@@ -363,6 +364,77 @@ bool lr_fast_plan(const attnres_read_desc* d, const Plan& pl, bool backward, Fas
   return true;
 }
 
+// LR reads with the row split over the waves of a workgroup
+// (attnres_lr_split.h), for what lr_fast_plan refuses: a static query alone,
+// rows of up to 2048, head widths of whole 16-lane rows, key slices of 1, 2, 4,
+// 8 or 16 16-byte chunks.  items: (pair, chunk) items per wave of the backward,
+// which holds four per lane.
+// Grids, us at 16384 tokens of d768 (N 13) / d1024 (N 13) / at 8192 of d1024 (N 25),
+// one head: forward 2048 / 4096 / 8192 / 16384 workgroups 92, 98, 107 / 86, 101,
+// 101 / 85, 99, 98 / 89, 98, 98; backward 1024 / 1536 / 2048 / 4096 150, 190,
+// 189 / 166, 190, 194 / 157, 204, 199 / 154, 192, 190.
+constexpr int kLrSplitFwdGroups = 8192;
+struct LrSplitPlan {
+  int vb, wpt, nb, nh, np, kch, ki;
+};
+
+bool lr_split_plan(const attnres_read_desc* d, const Plan& pl, bool backward, LrSplitPlan* f) {
+  if (!pl.lr || !pl.vec || !pl.key_vec) return false;
+  if (!d->query || d->query_dyn || d->gate || d->static_keys) return false;
+  const int es = elem_size(d->dtype), N = d->n_src, D = d->dim, H = d->heads, dh = D / H;
+  // 16-byte vectors where whole waves of them cover the row and the sources
+  // fit the registers, 8-byte ones otherwise (16-bit types): d1024 N 13 forward
+  // 99 against 112 us, backward 192 against 204; d2048 N 9 37 / 75 against 46 / 84
+  f->vb = es == 4 || (D % 512 == 0 && dh % 128 == 0 && N <= 32) ? 16 : 8;
+  if (es == 4 && N > 32) return false;
+  const int E = f->vb / es, colw = kWaveSize * E;
+  if (D > 2048 || D % E || dh % (16 * E) || H > 255) return false;
+  f->wpt = (D + colw - 1) / colw;
+  f->nb = lr_split_slots(N);
+  f->np = 2;
+  while (f->np < N) f->np <<= 1;
+  const int rh = d->rank / H;
+  f->kch = rh * es / 16;
+  if ((rh * es) % 16 || f->kch > 16 || (f->kch & (f->kch - 1))) return false;
+  f->nh = 0;
+  int items = 0;
+  for (int w = 0; w < f->wpt; ++w) {
+    const int c0 = w * colw, c1 = c0 + colw < D ? c0 + colw : D;
+    const int nh = (c1 - 1) / dh - c0 / dh + 1;
+    if (nh > f->nh) f->nh = nh;
+    const int pr = (int)((int64_t)H * N * c1 / D - (int64_t)H * N * c0 / D);
+    if (pr * f->kch > items) items = pr * f->kch;
+  }
+  f->ki = items <= kWaveSize ? 1 : 4;
+  if (backward && items > 4 * kWaveSize) return false;
+  // 32-bit token index and byte strides in the row addresses
+  if (d->n_tok > INT32_MAX) return false;
+  for (int s = 0; s < N; ++s)
+    if ((uint64_t)d->value_row_stride[s] * es > UINT32_MAX || (uint64_t)d->key_row_stride[s] * es > UINT32_MAX)
+      return false;
+  return true;
+}
+
+size_t lr_split_lds_bytes(const attnres_read_desc* d, const LrSplitPlan& f, bool backward) {
+  const int HN = d->heads * d->n_src;
+  size_t b = lr_split_lds_head(d->rank, elem_size(d->dtype), HN, f.wpt, f.nh, f.np) + 16 * sizeof(float);
+  if (backward) {
+    const size_t dw = 2 * 4 * (size_t)f.wpt * d->n_src, fold = (size_t)HN * (d->rank / d->heads + 1);
+    b += (dw > fold ? dw : fold) * sizeof(float);
+  }
+  return b;
+}
+
+void fill_lr_split(const LrSplitPlan& f, ReadParams* p, Launch* L) {
+  p->nh = f.nh;
+  p->np = f.np;
+  p->kch = f.kch;
+  L->vb = f.vb;
+  L->wpt = f.wpt;
+  L->nmax = f.nb;
+  L->teams = f.ki;
+}
+
 // Base-key fast path (attnres_base_fast.h): 16-bit rows that one wave covers
 // exactly with 8-byte (D = 256, 768) or 16-byte (D = 512, 1024) lane vectors,
 // up to 16 sources, no output norm.  vb / cb / nb = vector bytes, columns per
@@ -552,6 +624,11 @@ extern "C" int attnres_read_forward(const attnres_read_desc* d, void* out, void*
               4 * (size_t)lr_fast_staged_rows(f.cb, f.rhc, f.nb, elem_size(d->dtype), lr_fast_features(d)) * 1024;
       if (L.lds > lds_limit()) return fail(ATTNRES_EUNSUPPORTED, "LR forward needs %zu bytes of LDS", L.lds);
       err = launch_lr_fast_forward(d->dtype, p, L, st);
+    } else if (LrSplitPlan sp; lr_split_plan(d, pl, false, &sp)) {
+      fill_lr_split(sp, &p, &L);
+      L.grid = (int)(d->n_tok < kLrSplitFwdGroups ? d->n_tok : kLrSplitFwdGroups);
+      L.lds = lr_split_lds_bytes(d, sp, false);
+      err = launch_lr_split_forward(d->dtype, p, L, st);
     } else {
       L.lds = (2 * (size_t)d->heads * d->n_src + 32) * sizeof(float);
       if (L.lds > lds_limit()) return fail(ATTNRES_EUNSUPPORTED, "LDS need %zu bytes", L.lds);
@@ -715,6 +792,12 @@ extern "C" int attnres_read_backward(const attnres_read_desc* d, const attnres_r
       // beats 16-slot tiles here, measured at C3 and C4)
       partials_layout = kPartSlotMajor;
       err = launch_lr_fast_backward(d->dtype, bp, L, st);
+    } else if (LrSplitPlan sp; lr_split_plan(d, pl, true, &sp) && lr_split_lds_bytes(d, sp, true) <= lds_limit()) {
+      fill_lr_split(sp, &bp.f, &L);
+      L.grid = (int)groups;
+      L.lds = lr_split_lds_bytes(d, sp, true);
+      partials_layout = kPartSlotMajor;
+      err = launch_lr_split_backward(d->dtype, bp, L, st);
     } else {
       L.lds = lr_bwd_lds(d, pl, PL.n_part);
       if (L.lds > lds_limit())

@@ -32,6 +32,11 @@ hipError_t launch_value_norm(int dtype, bool bwd, const ValueNormParams& p, int 
 // L.nmax = source slots (8/16/32), L.teams = key chunks per head slot (2/8)
 hipError_t launch_lr_fast_forward(int dtype, const ReadParams& p, const Launch& L, hipStream_t st);
 hipError_t launch_lr_fast_backward(int dtype, const ReadBwdParams& p, const Launch& L, hipStream_t st);
+// LR reads with a token's row split over the L.wpt waves of a workgroup
+// (attnres_lr_split.h): L.vb = vector bytes, L.nmax = source slots, backward
+// L.teams = key-gradient items per lane (1/4)
+hipError_t launch_lr_split_forward(int dtype, const ReadParams& p, const Launch& L, hipStream_t st);
+hipError_t launch_lr_split_backward(int dtype, const ReadBwdParams& p, const Launch& L, hipStream_t st);
 size_t lr_fast_table_bytes();  // LDS bytes of the fast kernels' per-source tables
 // base-key fast path (one wave per token, 16-bit rows of 256 / 512 / 768 / 1024):
 // L.vb = vector bytes (8/16), L.wpt = columns per lane, L.nmax = source slots

@@ -481,6 +481,32 @@ bool base_fast_plan(const attnres_read_desc* d, const Plan& pl, BaseFastPlan* f)
   return true;
 }
 
+// Base reads with the row split over the waves of a workgroup
+// (attnres_base_split.h): rows of up to 2048 elements.  16-bit types: the
+// forward in 16-byte vectors where whole waves of them cover the row and the
+// sources fit the registers (d1024 N 9, output norm, 16384 tokens: 67 against
+// 71 us with 8-byte ones), else in 8-byte ones; the backward always in 8-byte
+// ones, at twice the waves and half the registers (the same read: 149 against
+// 161 us; N 25, 8192 tokens: 203 against 242).
+struct BaseSplitPlan {
+  int vb, wpt, nb;
+};
+
+bool base_split_plan(const attnres_read_desc* d, const Plan& pl, bool backward, BaseSplitPlan* f) {
+  if (d->mode != ATTNRES_MODE_SOFTMAX || pl.lr || !pl.vec || !d->query) return false;
+  const int es = elem_size(d->dtype), N = d->n_src, D = d->dim;
+  if (D > 2048 || (es == 4 && N > 32)) return false;
+  f->vb = es == 4 || (!backward && D % 512 == 0 && N <= 32) ? 16 : 8;
+  const int colw = kWaveSize * (f->vb / es);
+  f->wpt = (D + colw - 1) / colw;
+  f->nb = lr_split_slots(N);
+  // 32-bit token index and byte strides in the row addresses
+  if (d->n_tok > INT32_MAX) return false;
+  for (int s = 0; s < N; ++s)
+    if ((uint64_t)d->value_row_stride[s] * es > UINT32_MAX) return false;
+  return true;
+}
+
 // Optional code the fast LR kernels must carry for a read, rounded up to an
 // instantiated set: 0 (static query, no output norm), kFeatDyn (per-token query
 // / gate), kFeatDyn | kFeatStatic (and static source keys) or kFeatAll.
@@ -645,6 +671,12 @@ extern "C" int attnres_read_forward(const attnres_read_desc* d, void* out, void*
       L.grid = (int)((p.streams + 3) / 4);
       L.lds = lr_fast_table_bytes();
       err = launch_base_fast_forward(d->dtype, p, L, st);
+    } else if (BaseSplitPlan sp; base_split_plan(d, pl, false, &sp)) {
+      L.vb = sp.vb;
+      L.wpt = sp.wpt;
+      L.nmax = sp.nb;
+      L.grid = (int)(d->n_tok < kLrSplitFwdGroups ? d->n_tok : kLrSplitFwdGroups);
+      err = launch_base_split_forward(d->dtype, p, L, st);
     } else {
       L.lds = (pl.nmax <= 16 ? (size_t)pl.wpt * pl.nmax + 32 : (size_t)d->n_src + 32) * sizeof(float);
       err = launch_base_forward(d->dtype, p, L, st);
@@ -824,6 +856,16 @@ extern "C" int attnres_read_backward(const attnres_read_desc* d, const attnres_r
         (size_t)L.grid * part_stride(PL.n_part) <= (size_t)groups * PL.n_part ? kPartTiled : kPartSlotMajor;
     bp.part_layout = partials_layout;
     err = launch_base_fast_backward(d->dtype, bp, L, st);
+  } else if (BaseSplitPlan sp; base_split_plan(d, pl, true, &sp)) {
+    L.vb = sp.vb;
+    L.wpt = sp.wpt;
+    L.nmax = sp.nb;
+    L.grid = (int)full_groups;  // d1024 N 9 / d640 N 7, 1024 / 1280 / 2048 workgroups: 160, 57 / 154, 51 / 149, 50 us
+    // (as the fast backward: tiles unless they would not fit the workspace)
+    partials_layout =
+        (size_t)L.grid * part_stride(PL.n_part) <= (size_t)groups * PL.n_part ? kPartTiled : kPartSlotMajor;
+    bp.part_layout = partials_layout;
+    err = launch_base_split_backward(d->dtype, bp, L, st);
   } else {
     size_t fl = pl.nmax <= 16 ? (size_t)pl.wpt * pl.nmax + 32 : 2 * (size_t)d->n_src + 32;
     if ((size_t)L.teams * PL.n_part > fl) fl = (size_t)L.teams * PL.n_part;

@@ -37,6 +37,9 @@ hipError_t launch_lr_fast_backward(int dtype, const ReadBwdParams& p, const Laun
 // L.teams = key-gradient items per lane (1/4)
 hipError_t launch_lr_split_forward(int dtype, const ReadParams& p, const Launch& L, hipStream_t st);
 hipError_t launch_lr_split_backward(int dtype, const ReadBwdParams& p, const Launch& L, hipStream_t st);
+// base reads split the same way (attnres_base_split.h)
+hipError_t launch_base_split_forward(int dtype, const ReadParams& p, const Launch& L, hipStream_t st);
+hipError_t launch_base_split_backward(int dtype, const ReadBwdParams& p, const Launch& L, hipStream_t st);
 size_t lr_fast_table_bytes();  // LDS bytes of the fast kernels' per-source tables
 // base-key fast path (one wave per token, 16-bit rows of 256 / 512 / 768 / 1024):
 // L.vb = vector bytes (8/16), L.wpt = columns per lane, L.nmax = source slots

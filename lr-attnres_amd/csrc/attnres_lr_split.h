@@ -39,11 +39,10 @@ namespace attnres {
 // Source slots: instantiated counts, and the smallest source count each holds
 // (slots below it need no guard).
 __host__ __device__ constexpr int lr_split_slots(int n) {
-  return n <= 4 ? 4 : n <= 6 ? 6 : n <= 8 ? 8 : n <= 10 ? 10 : n <= 12 ? 12 : n <= 14 ? 14 : n <= 16 ? 16 : n <= 20 ? 20
-         : n <= 24 ? 24 : n <= 28 ? 28 : n <= 32 ? 32 : n <= 40 ? 40 : n <= 48 ? 48 : n <= 56 ? 56 : 64;
+  return n <= 4 ? 4 : n <= 32 ? (n + 1) / 2 * 2 : (n + 3) / 4 * 4;
 }
 __host__ __device__ constexpr int lr_split_floor(int nb) {
-  return nb <= 4 ? 1 : nb <= 16 ? nb - 1 : nb <= 32 ? nb - 3 : nb - 7;
+  return nb <= 4 ? 1 : nb <= 32 ? nb - 1 : nb - 3;
 }
 
 // Per-wave column ownership and the workgroup's LDS carve-up, shared by both
@@ -445,8 +444,9 @@ __global__ void __launch_bounds__(512) lr_split_bwd_kernel(const ReadBwdParams b
 
 // launch switch: L.nmax = source slots, L.vb = vector bytes (8 / 16); 16-byte
 // vectors hold up to 32 sources
-#define ATTNRES_LR_SPLIT_NB8(CASE) CASE(40) CASE(48) CASE(56) CASE(64)
+#define ATTNRES_LR_SPLIT_NB8(CASE) CASE(36) CASE(40) CASE(44) CASE(48) CASE(52) CASE(56) CASE(60) CASE(64)
 #define ATTNRES_LR_SPLIT_NB(CASE) \
-  CASE(4) CASE(6) CASE(8) CASE(10) CASE(12) CASE(14) CASE(16) CASE(20) CASE(24) CASE(28) CASE(32)
+  CASE(4) CASE(6) CASE(8) CASE(10) CASE(12) CASE(14) CASE(16) CASE(18) CASE(20) CASE(22) CASE(24) CASE(26) CASE(28) \
+  CASE(30) CASE(32)
 
 }  // namespace attnres

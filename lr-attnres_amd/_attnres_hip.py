@@ -8,6 +8,7 @@ There is no CPU path: a missing library or a non-GPU tensor raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 from ctypes import POINTER, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p
 
@@ -15,6 +16,7 @@ import torch
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libattnres_hip.so")
+NATIVE_PATH = os.path.join(HERE, "_attnres_torch.so")
 
 ABI_VERSION = 9
 MAX_SOURCES = 64
@@ -320,6 +322,25 @@ def load() -> ctypes.CDLL:
         raise RuntimeError(f"libattnres_hip ABI {v} != expected {ABI_VERSION}; rebuild the library")
     _lib = lib
     return lib
+
+
+_native = None
+
+
+def native():
+    """The C++ host side of the eager calls (csrc/attnres_torch.cpp), bound to the library; raises when it is not built."""
+    global _native
+    if _native is None:
+        load()
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError(f"attnres host extension not found at {NATIVE_PATH}; build it with "
+                               "`python lr-attnres_amd/build.py` (or __graft_entry__.build())")
+        spec = importlib.util.spec_from_file_location("_attnres_torch", NATIVE_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.bind(LIB_PATH)
+        _native = mod
+    return _native
 
 
 def available() -> bool:

@@ -49,6 +49,7 @@ __all__ = [
 ]
 
 _ALLOWED = (torch.float32, torch.bfloat16, torch.float16)
+_GATE_ACTS = {"linear": _hip.GATE_LINEAR, "sigmoid": _hip.GATE_SIGMOID}
 
 
 def is_fused_attnres_available() -> bool:
@@ -330,6 +331,42 @@ def _compiling() -> bool:
     return torch.compiler.is_compiling()
 
 
+# The C++ host side (csrc/attnres_torch.cpp) takes the plain eager calls: it
+# answers None, with nothing launched, for whatever needs a conversion, a copy
+# or an error message, and the code below it in each function then runs.  So
+# does a call whose Python binding has been replaced (a recorder, a test's spy):
+# what replaces it is called.
+_NATIVE = None
+_BOUND = {name: getattr(_hip, name) for name in (
+    "forward", "backward", "phase1_forward", "phase1_backward_sites", "phase1_bank_forward", "phase1_bank_backward",
+    "phase2_forward", "phase2_backward", "accum_read_forward", "accum_read_backward", "block_accum_forward",
+    "block_accum_backward")}
+
+
+def _native(fwd: str, bwd: str):
+    global _NATIVE
+    if _NATIVE is None:
+        _NATIVE = _hip.native() if torch.cuda.is_available() else False
+    if _NATIVE is False or _compiling():
+        return None
+    return _NATIVE if getattr(_hip, fwd) is _BOUND[fwd] and getattr(_hip, bwd) is _BOUND[bwd] else None
+
+
+def _native_bias(source_counts, source_logit_biases, values):
+    """(whether the native call can take the logit bias, the bias)."""
+    if source_counts is None and source_logit_biases is None:
+        return True, None
+    if isinstance(source_logit_biases, Tensor):
+        return source_counts is None, source_logit_biases
+    n = len(values)
+    given = source_logit_biases if source_counts is None else source_counts
+    if n == 0 or not isinstance(given, (list, tuple)) or len(given) != n or not isinstance(values, (list, tuple)):
+        return False, None
+    if not all(type(x) in (float, int) for x in given) or not values[0].is_cuda:
+        return False, None
+    return True, _source_logit_bias(source_counts, source_logit_biases, n, values[0].device)
+
+
 def _device_ctx(dev):
     """Device guard, skipped when ``dev`` is already the current device."""
     return contextlib.nullcontext() if dev.index == torch.cuda.current_device() else torch.cuda.device(dev)
@@ -416,6 +453,13 @@ def attention_residual_read(values, query: Tensor, key_norm: bool, force_triton:
     Keys are ``rms_norm(values)`` when ``key_norm``.  A single source is
     returned as is (rms-normed when ``normalize_output``).
     """
+    nat = _native("forward", "backward")
+    if nat:
+        ok, bias = _native_bias(source_counts, source_logit_biases, values)
+        out = nat.read(values, None, query, None, None, bias, None, 1, 1.0, bool(key_norm), bool(normalize_output),
+                       _hip.GATE_NONE) if ok else None
+        if out is not None:
+            return out
     srcs = _sources(values)
     _check_sources(srcs, "attention_residual_read")
     if len(srcs) == 1:
@@ -508,6 +552,14 @@ def lrid_attention_residual_read(values, keys, query: Tensor, num_heads: int, lo
     parameter cast to the key dtype in every other row; autograd then sums the
     rows' gradients back into the parameter.
     """
+    nat = _native("forward", "backward")
+    if nat and type(num_heads) is int and isinstance(query, Tensor):
+        ok, bias = _native_bias(source_counts, source_logit_biases, values)
+        q = (None, query) if query.dim() == 4 else (query, None)
+        out = nat.read(values, keys, *q, None, bias, static_keys, num_heads, float(logit_scale), bool(key_norm),
+                       bool(normalize_output), _hip.GATE_NONE) if ok else None
+        if out is not None:
+            return out
     vs, ks, H, D, R, k0_dtype = _lr_common(values, keys, num_heads, "lrid_attention_residual_read")
     query = query.to(k0_dtype)
     if len(vs) == 1:
@@ -553,6 +605,14 @@ def lrid_attention_residual_read_gated(values, keys, static_query: Optional[Tens
     eagerly and then reads with an input-dependent query.  ``static_keys`` as
     in ``lrid_attention_residual_read`` (config 4's [N, 128] static source key).
     """
+    nat = _native("forward", "backward")
+    if nat and type(num_heads) is int and gate_activation in _GATE_ACTS:
+        ok, bias = _native_bias(source_counts, source_logit_biases, values)
+        out = nat.read(values, keys, static_query, dynamic_query, gate, bias, static_keys, num_heads,
+                       float(logit_scale), bool(key_norm), bool(normalize_output),
+                       _GATE_ACTS[gate_activation] if gate is not None else _hip.GATE_NONE) if ok else None
+        if out is not None:
+            return out
     vs, ks, H, D, R, _ = _lr_common(values, keys, num_heads, "lrid_attention_residual_read_gated")
     dtype = vs[0].dtype
     B, T, _ = vs[0].shape
@@ -566,7 +626,7 @@ def lrid_attention_residual_read_gated(values, keys, static_query: Optional[Tens
         if static_query.numel() != R:
             raise RuntimeError(f"static_query must have {R} elements")
         qs = static_query.to(dtype).reshape(H, R // H).contiguous()
-    act = {"linear": _hip.GATE_LINEAR, "sigmoid": _hip.GATE_SIGMOID}.get(gate_activation)
+    act = _GATE_ACTS.get(gate_activation)
     if act is None:
         raise RuntimeError(f"unknown gate_activation {gate_activation!r}")
     g = None
@@ -785,6 +845,11 @@ def lrid_block_phase1(values, source_logits):
     ``attnres_ops.py:3910-3961``), with the stack and its backward's slices
     left out.
     """
+    nat = _native("phase1_forward", "phase1_backward_sites")
+    if nat:
+        res = nat.phase1_sources(values, source_logits)
+        if res is not None:
+            return res
     srcs = _promote(_sources(values))
     S = len(srcs)
     if S == 0 or len(source_logits) != S:
@@ -958,6 +1023,11 @@ def attention_residual_phase1(values, queries: Tensor, key_norm: bool, force_tri
     keyed-logits kernels and read over them with
     ``attention_residual_phase1_from_logits``.  Returns (out [Q,B,T,D], lse [Q,B,T]).
     """
+    nat = _native("phase1_bank_forward", "phase1_bank_backward")
+    if nat:
+        res = nat.phase1_bank(values, queries, bool(key_norm))
+        if res is not None:
+            return res
     srcs = _sources(values)
     if len(srcs) == 0:
         raise RuntimeError("Two-phase AttnRes phase1 requires at least one source")
@@ -1134,6 +1204,16 @@ def _scalar_arg(x, device, what):
 
 def _phase2(partial_value, partial_key, query, partial_logit, interblock_output, interblock_lse, merge, key_norm,
             normalize_output, logit_scale, logit_bias, partial_scale, scale_key, what, query_row=None):
+    nat = _native("phase2_forward", "phase2_backward")
+    if (nat and partial_logit is None and type(logit_bias) in (float, int)
+            and (partial_scale is None or type(partial_scale) in (float, int))
+            and (query_row is None or type(query_row) is int and query_row >= 0)):
+        out = nat.phase2(partial_value, partial_key, query, interblock_output, interblock_lse, int(merge),
+                         bool(key_norm), bool(normalize_output), float(logit_scale), float(logit_bias),
+                         1.0 if partial_scale is None else float(partial_scale), bool(scale_key),
+                         -1 if query_row is None else query_row)
+        if out is not None:
+            return out
     if partial_value.dim() != 3:
         raise RuntimeError(f"{what}: partial_value must be [B, T, D]")
     B, T, D = partial_value.shape
@@ -1509,6 +1589,13 @@ def lrid_block_accumulate(projected: Tensor, partial_value: Optional[Tensor], pa
     sublayer of a block.  Every add and product rounds to the dtype as the
     eager ops do.  Returns ``(value [..., D], key [..., rank])``.
     """
+    nat = _native("block_accum_forward", "block_accum_backward")
+    if (nat and not value_norm and not scale_key and type(partial_scale) in (float, int)
+            and (complete or partial_scale == 1.0)):
+        res = nat.block_accum(projected, partial_value, partial_key, int(output_dim), int(rank), int(num_heads),
+                              bool(key_norm), bool(complete), float(partial_scale))
+        if res is not None:
+            return res
     P = projected.size(-1)
     if P < output_dim + rank:
         raise RuntimeError(f"lrid_block_accumulate: projection has {P} columns, needs at least {output_dim + rank}")
@@ -1637,6 +1724,16 @@ def lrid_block_accumulate_read(projected: Tensor, partial_value: Optional[Tensor
     """
     mkn = key_norm if merge_key_norm is None else bool(merge_key_norm)
     D, R = int(output_dim), int(rank)
+    nat = _native("accum_read_forward", "accum_read_backward")
+    if (nat and type(query_row) is int and type(logit_bias) in (float, int)
+            and (partial_scale is None or type(partial_scale) in (float, int))):
+        res = nat.accum_read(projected, partial_value, partial_key, query, interblock_output, interblock_lse, D, R,
+                             float(logit_scale), int(num_heads), bool(key_norm), mkn,
+                             _hip.MERGE_LERP if lerp else _hip.MERGE_ADDCMUL, bool(normalize_output),
+                             float(logit_bias), 1.0 if partial_scale is None else float(partial_scale),
+                             bool(scale_key), query_row)
+        if res is not None:
+            return res
     if interblock_output.dim() != 3 or interblock_output.size(-1) != D:
         raise RuntimeError(f"lrid_block_accumulate_read: interblock_output must be [B, T, {D}]")
     B, T = interblock_output.shape[:2]

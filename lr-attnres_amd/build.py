@@ -1,4 +1,5 @@
-"""Build libattnres_hip.so (gfx950) in-tree from lr-attnres_amd/csrc/*.hip.
+"""Build libattnres_hip.so (gfx950) in-tree from lr-attnres_amd/csrc/*.hip, and the
+host extension _attnres_torch.so (csrc/attnres_torch.cpp, against torch's C++ headers).
 
     python lr-attnres_amd/build.py [--arch gfx950] [--jobs 4]
 
@@ -19,6 +20,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libattnres_hip.so")
+EXT = os.path.join(HERE, "_attnres_torch.so")
 
 SOURCES = ["attnres_capi.hip", "attnres_lr.hip", "attnres_lr_fast_fwd.hip", "attnres_lr_fast_bwd.hip",
            "attnres_lr_split_fwd.hip", "attnres_lr_split_bwd.hip", "attnres_lr_split_bwd8.hip",
@@ -48,10 +50,35 @@ def compile_one(src: str, arch: str) -> str:
     return obj
 
 
+def build_ext() -> str:
+    """The host extension: plain C++ over torch's headers and the C ABI's (no device code)."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    tmp = EXT + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-DUSE_ROCM",
+           "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    for inc in (*include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]):
+        cmd += ["-isystem", inc]
+    cmd += [os.path.join(CSRC, "attnres_torch.cpp"), "-o", tmp]
+    for lib in library_paths():
+        cmd += ["-L", lib]
+    cmd += ["-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-ldl"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"host extension failed:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, EXT)
+    return EXT
+
+
 def build(arch: str = "gfx950", jobs: int = 4, verbose: bool = False) -> str:
     os.makedirs(BUILD, exist_ok=True)
     with cf.ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
+        ext = ex.submit(build_ext)
         objs = list(ex.map(lambda s: compile_one(s, arch), SOURCES))
+        ext.result()
     tmp = LIB + ".tmp"
     cmd = [_hipcc(), f"--offload-arch={arch}", "-shared", "-fPIC", *objs, "-o", tmp]
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -59,7 +86,7 @@ def build(arch: str = "gfx950", jobs: int = 4, verbose: bool = False) -> str:
         raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, LIB)
     if verbose:
-        print(f"built {LIB}")
+        print(f"built {LIB} and {EXT}")
     return LIB
 
 

@@ -311,6 +311,17 @@ def load() -> ctypes.CDLL:
     lib.attnres_value_norm_backward.restype = c_int
     lib.attnres_value_norm_backward.argtypes = [POINTER(ValueKeyDesc), c_void_p, POINTER(c_float),
                                                 POINTER(c_void_p), c_void_p]
+    lib.attnres_value_keys_fits.restype = c_int
+    lib.attnres_value_keys_fits.argtypes = [POINTER(ValueKeyDesc), c_int32]
+    lib.attnres_value_keys_forward.restype = c_int
+    lib.attnres_value_keys_forward.argtypes = [POINTER(ValueKeyDesc), c_void_p, c_int32, c_void_p, POINTER(c_float),
+                                               c_void_p]
+    lib.attnres_value_keys_backward_workspace_size.restype = c_size_t
+    lib.attnres_value_keys_backward_workspace_size.argtypes = [POINTER(ValueKeyDesc), c_int32]
+    lib.attnres_value_keys_backward.restype = c_int
+    lib.attnres_value_keys_backward.argtypes = [POINTER(ValueKeyDesc), c_void_p, c_int32, POINTER(c_void_p), c_void_p,
+                                                POINTER(c_float), POINTER(c_void_p), c_void_p, c_void_p, c_size_t,
+                                                c_void_p]
     lib.attnres_kernel_timing.restype = c_int
     lib.attnres_kernel_timing.argtypes = [c_int]
     lib.attnres_test_phase2_block_layout.restype = c_int
@@ -1053,3 +1064,36 @@ def value_norm_backward(d: ValueKey, device, dtype, grad_normed, inv, lead):
                                          _stream(device))
     _check(rc, "value norm backward")
     return dvals
+
+
+def value_keys_fits(d: ValueKey, weight) -> bool:
+    """Whether the fused value-key projection takes these sources and this weight (include/attnres_value_keys.h)."""
+    return (weight.is_contiguous() and weight.data_ptr() % 16 == 0
+            and bool(load().attnres_value_keys_fits(ctypes.byref(d.c), int(weight.size(0)))))
+
+
+def value_keys_forward(d: ValueKey, weight, for_backward: bool):
+    """(keys [N, n_tok, R], inv_rms [N, n_tok] | None)."""
+    R = weight.size(0)
+    keys = torch.empty((d.n_src, d.n_tok, R), device=weight.device, dtype=weight.dtype)
+    inv = torch.empty((d.n_src, d.n_tok), device=weight.device, dtype=torch.float32) if for_backward else None
+    rc = load().attnres_value_keys_forward(ctypes.byref(d.c), _ptr(weight), R, _ptr(keys), _fptr(inv),
+                                           _stream(weight.device))
+    _check(rc, "value keys forward")
+    return keys, inv
+
+
+def value_keys_backward(d: ValueKey, weight, grad_keys, keys, inv_rms, want_values: bool, want_weight: bool, lead):
+    """(dvalues list of lead + [D] | None, dweight [R, D] | None); grad_keys: N dense [n_tok, R] tensors or None each."""
+    lib = load()
+    n, R, dev = d.n_src, weight.size(0), weight.device
+    dvals = _row_blocks(n, d.n_tok, d.D, dev, weight.dtype, True, lead) if want_values else None
+    dw = torch.empty_like(weight) if want_weight else None
+    gk = (c_void_p * n)(*[g.data_ptr() if g is not None else None for g in grad_keys])
+    dv = (c_void_p * n)(*[t.data_ptr() for t in dvals]) if want_values else None
+    ws_bytes = lib.attnres_value_keys_backward_workspace_size(ctypes.byref(d.c), R)
+    ws = torch.empty((max(1, ws_bytes),), device=dev, dtype=torch.uint8)
+    rc = lib.attnres_value_keys_backward(ctypes.byref(d.c), _ptr(weight), R, gk, _ptr(keys), _fptr(inv_rms), dv,
+                                         _ptr(dw), _ptr(ws), ws_bytes, _stream(dev))
+    _check(rc, "value keys backward")
+    return dvals, dw

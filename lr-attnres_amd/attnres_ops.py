@@ -1491,17 +1491,49 @@ class _ValueKeyFn(torch.autograd.Function):
         return (None, dw) + tuple(dv if want[2 + i] else None for i, dv in enumerate(dvals))
 
 
+class _ValueKeyGemmFn(torch.autograd.Function):
+    """Eager autograd of the value-derived keys with their projection in one kernel each way: inputs (W [R, D], *values);
+    outputs N keys [B, T, R]."""
+
+    @staticmethod
+    def forward(ctx, weight, *values):
+        B, T, _ = values[0].shape
+        n, R = len(values), weight.size(0)
+        ctx.set_materialize_grads(False)
+        with _device_ctx(weight.device):
+            keys, inv = _hip.value_keys_forward(_hip.ValueKey(values), weight, any(ctx.needs_input_grad))
+        # the keys' rows serve the norm's backward; as one block of its own, not as the outputs
+        ctx.save_for_backward(weight, keys, inv, *values)
+        return tuple(keys.view(n, B, T, R).unbind(0))
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, *grad_keys):
+        weight, keys, inv, *values = ctx.saved_tensors
+        n, (B, T, _), R = len(values), values[0].shape, weight.size(0)
+        if all(g is None for g in grad_keys):
+            return (None,) * (1 + n)
+        gk = [None if g is None else g.reshape(B * T, R).contiguous() for g in grad_keys]
+        gk = [g.clone() if g is not None and g.data_ptr() % 16 else g for g in gk]  # (views into larger gradients)
+        want = ctx.needs_input_grad
+        with _device_ctx(weight.device):
+            dvals, dw = _hip.value_keys_backward(_hip.ValueKey(values), weight, gk, keys, inv, any(want[1:]), want[0],
+                                                 (B, T))
+        return (dw, *[dvals[i] if want[1 + i] else None for i in range(n)])
+
+
 def lrid_value_key_projection(values, weight: Tensor, value_norm: bool = True):
     """LR keys projected from the sources' values: ``rms_norm(v_s) @ W^T``.
 
     Not in the reference's op module: the reference's
     ``LRIDSourceKeyProjection.forward`` (model.py:420-428, with
     ``lrid_key_from_value`` and ``lrid_key_value_norm``) does this per source as
-    ``self.proj(norm(x))`` -- config 4's key producer.  Here one HIP pass
-    rms-norms every source (fp32, one rounding to the dtype) into one block, a
-    single library GEMM projects all of them, and the backward runs the GEMMs
-    for the weight and input gradients and one HIP pass of the rms-norm
-    backward.  ``values``: N x [B, T, D] (or [N, B, T, D]); ``weight`` [R, D]
+    ``self.proj(norm(x))`` -- config 4's key producer.  Here bf16 rows of a
+    multiple of 64 up to 4096 with rank 32, 64 or 128 take one matrix-core kernel
+    each way (the normed rows never leave the registers); other forms rms-norm
+    every source in one HIP pass (fp32, one rounding to the dtype) into one block,
+    project all of them with a single library GEMM, and run the GEMMs for the
+    weight and input gradients and one HIP pass of the rms-norm backward.  ``values``: N x [B, T, D] (or [N, B, T, D]); ``weight`` [R, D]
     (``nn.Linear(D, R).weight``).  Returns N keys [B, T, R] in the values' dtype.
     """
     vs = _sources(values)
@@ -1513,6 +1545,8 @@ def lrid_value_key_projection(values, weight: Tensor, value_norm: bool = True):
         raise RuntimeError(f"lrid_value_key_projection: weight must be [rank, {D}], got {tuple(weight.shape)}")
     vs = [_hip.as_rows(t) for t in vs]
     w = weight.to(vs[0].dtype)
+    if value_norm and not _compiling() and _hip.value_keys_fits(_hip.ValueKey(vs), w):
+        return list(_ValueKeyGemmFn.apply(w, *vs))
     return list(_ValueKeyFn.apply((bool(value_norm),), w, *vs))
 
 

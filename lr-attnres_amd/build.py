@@ -27,7 +27,7 @@ SOURCES = ["attnres_capi.hip", "attnres_lr.hip", "attnres_lr_fast_fwd.hip", "att
            "attnres_base_split_fwd.hip", "attnres_base_split_bwd.hip",
            "attnres_base.hip", "attnres_base_bwd.hip",
            "attnres_base_fast_fwd.hip", "attnres_base_fast_bwd.hip", "attnres_phase1.hip", "attnres_phase1_fast.hip", "attnres_phase1_bank.hip", "attnres_phase2.hip", "attnres_phase2_fast.hip", "attnres_keysplit.hip",
-           "attnres_keyed_logits.hip", "attnres_value_key.hip", "attnres_site_logits.hip"]
+           "attnres_keyed_logits.hip", "attnres_value_key.hip", "attnres_value_gemm.hip", "attnres_site_logits.hip"]
 
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 

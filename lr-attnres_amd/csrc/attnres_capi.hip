@@ -10,6 +10,7 @@
 #include <string>
 
 #include "../../include/attnres_phase1_bank.h"
+#include "../../include/attnres_value_keys.h"
 #include "attnres_launch.h"
 #include "attnres_lr_split.h"
 #include "attnres_params.h"
@@ -2329,5 +2330,117 @@ extern "C" int attnres_value_norm_backward(const attnres_value_key_desc* d, cons
   p.inv = const_cast<float*>(inv_rms);
   hipError_t err = launch_value_norm(d->dtype, true, p, value_norm_grid(d), vec, (hipStream_t)stream);
   if (err != hipSuccess) return fail(ATTNRES_ELAUNCH, "value norm backward launch failed: %s", hipGetErrorString(err));
+  return ATTNRES_OK;
+}
+
+// ---------------------------------------------------------------- value-derived keys with their projection
+namespace {
+
+bool value_keys_ok(const attnres_value_key_desc* d, int rank) {
+  bool vec = false;
+  // bf16 only: rnd(inv gk) of a row of zeros (inv = 2896) would leave fp16's range
+  if (check_value_key(d, &vec) != ATTNRES_OK || d->n_tok < 1 || d->dtype != ATTNRES_DTYPE_BF16) return false;
+  if (rank != 32 && rank != 64 && rank != 128) return false;
+  if (d->dim % 64 || d->n_tok > INT32_MAX) return false;
+  for (int s = 0; s < d->n_src; ++s)
+    if (!aligned16(d->values[s]) || d->value_row_stride[s] % 8) return false;
+  return true;
+}
+
+// Token parts per source for dW: at most two workgroups (of two waves per SIMD) per
+// CU over the column groups and sources, parts of at least 256 tokens.  17 sources
+// of D = 2048, 3 / 4 / 5 / 7 parts: 389 / 439 / 374 / 358 us, but 10 / 12 / 15 / 20
+// for the reduction; 9 sources of D = 768, 18 / 20 / 25 / 35: 29 / 34 / 30 / 33.
+int value_keys_parts(const attnres_value_key_desc* d) {
+  const int64_t groups = (int64_t)((d->dim + 255) / 256) * d->n_src;
+  const int64_t want = groups < 512 ? 512 / groups : 1, most = (d->n_tok + 255) / 256;
+  return (int)(want < most ? want : most);
+}
+
+struct ValueKeysWork {
+  size_t wt, gs, c, partials, total;
+};
+ValueKeysWork value_keys_work(const attnres_value_key_desc* d, int rank) {
+  auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+  const size_t rows = (size_t)d->n_src * d->n_tok;
+  ValueKeysWork w;
+  w.wt = 0;
+  w.gs = up((size_t)d->dim * rank * 2);
+  w.c = w.gs + up(rows * rank * 2);
+  w.partials = w.c + up(rows * 4);
+  w.total = w.partials + (size_t)d->n_src * value_keys_parts(d) * rank * d->dim * 4;
+  return w;
+}
+
+void fill_value_keys(const attnres_value_key_desc* d, const void* weight, int rank, ValueKeysParams* p) {
+  memset(p, 0, sizeof(*p));
+  for (int s = 0; s < d->n_src; ++s) {
+    p->val[s] = d->values[s];
+    p->vstride[s] = (int32_t)d->value_row_stride[s];
+  }
+  p->weight = weight;
+  p->n_tok = d->n_tok;
+  p->n_src = d->n_src;
+  p->D = d->dim;
+  p->R = rank;
+  p->eps = d->norm_eps;
+}
+
+}  // namespace
+
+extern "C" int attnres_value_keys_fits(const attnres_value_key_desc* d, int32_t rank) {
+  return value_keys_ok(d, rank) ? 1 : 0;
+}
+
+extern "C" int attnres_value_keys_forward(const attnres_value_key_desc* d, const void* weight, int32_t rank, void* keys,
+                                          float* inv_rms, void* stream) {
+  if (!weight || !keys) return fail(ATTNRES_EINVAL, "weight / keys is NULL");
+  if (!value_keys_ok(d, rank) || !aligned16(weight) || !aligned16(keys))
+    return fail(ATTNRES_EUNSUPPORTED, "shape or alignment outside the value-key projection kernels");
+  ValueKeysParams p;
+  fill_value_keys(d, weight, rank, &p);
+  p.keys = keys;
+  p.inv = inv_rms;
+  hipError_t err = launch_value_keys(false, p, (hipStream_t)stream);
+  if (err != hipSuccess) return fail(ATTNRES_ELAUNCH, "value keys forward launch failed: %s", hipGetErrorString(err));
+  return ATTNRES_OK;
+}
+
+extern "C" size_t attnres_value_keys_backward_workspace_size(const attnres_value_key_desc* d, int32_t rank) {
+  return value_keys_ok(d, rank) ? value_keys_work(d, rank).total : 0;
+}
+
+extern "C" int attnres_value_keys_backward(const attnres_value_key_desc* d, const void* weight, int32_t rank,
+                                           const void* const* grad_keys, const void* keys, const float* inv_rms,
+                                           void* const* grad_values, void* grad_weight, void* workspace,
+                                           size_t workspace_bytes, void* stream) {
+  if (!weight || !grad_keys || !keys || !inv_rms) return fail(ATTNRES_EINVAL, "weight / grad_keys / keys / inv_rms is NULL");
+  if (!value_keys_ok(d, rank) || !aligned16(weight) || !aligned16(keys))
+    return fail(ATTNRES_EUNSUPPORTED, "shape or alignment outside the value-key projection kernels");
+  const ValueKeysWork w = value_keys_work(d, rank);
+  if (!workspace || workspace_bytes < w.total || !aligned16(workspace))
+    return fail(ATTNRES_EWORKSPACE, "workspace of %zu bytes needed, got %zu", w.total, workspace ? workspace_bytes : (size_t)0);
+  ValueKeysParams p;
+  fill_value_keys(d, weight, rank, &p);
+  for (int s = 0; s < d->n_src; ++s) {
+    if (!aligned16(grad_keys[s])) return fail(ATTNRES_EUNSUPPORTED, "grad_keys[%d] is not aligned to 16 bytes", s);
+    p.gkey[s] = grad_keys[s];
+    if (!grad_values) continue;
+    if (!grad_values[s]) return fail(ATTNRES_EINVAL, "grad_values[%d] is NULL", s);
+    if (!aligned16(grad_values[s])) return fail(ATTNRES_EUNSUPPORTED, "grad_values[%d] is not aligned to 16 bytes", s);
+    p.dval[s] = grad_values[s];
+  }
+  char* ws = (char*)workspace;
+  p.keys = const_cast<void*>(keys);
+  p.inv = const_cast<float*>(inv_rms);
+  p.wt = ws + w.wt;
+  p.gs = ws + w.gs;
+  p.c = (float*)(ws + w.c);
+  p.partials = (float*)(ws + w.partials);
+  p.dweight = grad_weight;
+  p.parts = value_keys_parts(d);
+  p.want_dv = grad_values != nullptr;
+  hipError_t err = launch_value_keys(true, p, (hipStream_t)stream);
+  if (err != hipSuccess) return fail(ATTNRES_ELAUNCH, "value keys backward launch failed: %s", hipGetErrorString(err));
   return ATTNRES_OK;
 }

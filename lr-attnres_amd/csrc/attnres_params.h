@@ -150,6 +150,25 @@ struct ValueNormParams {
   float eps;
 };
 
+// Value-derived keys with their projection (attnres_value_gemm.hip)
+struct ValueKeysParams {
+  const void* val[kMaxSources];
+  int32_t vstride[kMaxSources];  // row strides in elements
+  const void* gkey[kMaxSources]; // backward: [n_tok, R] dense, or null (zero)
+  void* dval[kMaxSources];       // backward: [n_tok, D] dense
+  const void* weight;            // [R, D] dense
+  void* keys;                    // [n_src, n_tok, R] dense (backward reads it)
+  float* inv;                    // [n_src, n_tok]
+  void* wt;                      // backward scratch: W^T [D, R]
+  void* gs;                      // backward scratch: rnd(inv gk) [n_src, n_tok, R]
+  float* c;                      // backward scratch: [n_src, n_tok]
+  float* partials;               // backward scratch: [n_src * parts][R, D]
+  void* dweight;                 // backward: [R, D], or null
+  int64_t n_tok;
+  int32_t n_src, D, R, parts, want_dv;
+  float eps;
+};
+
 struct ReduceParams {
   const float* partials;      // layout: kPart*
   int32_t n_groups, n_part;

@@ -62,7 +62,7 @@ hipError_t launch_phase1_split_forward(int dtype, const Phase1Params& p, const L
 hipError_t launch_phase1_split_backward(int dtype, const Phase1Params& p, const Launch& L, hipStream_t st);
 hipError_t launch_phase2_forward(int dtype, const Phase2Params& p, const Launch& L, hipStream_t st);
 hipError_t launch_phase2_backward(int dtype, const Phase2Params& p, const Launch& L, hipStream_t st);
-// phase 2 with base keys, 16-bit rows of 256 / 512 / 768 / 1024, no output norm:
+// phase 2 with base keys, 16-bit rows of 256 / 512 / 768 / 1024:
 // L.vb = vector bytes (8/16), L.wpt = columns per lane, L.feat bit 0 = key norm
 hipError_t launch_phase2_fast_forward(int dtype, const Phase2Params& p, const Launch& L, hipStream_t st);
 hipError_t launch_phase2_fast_backward(int dtype, const Phase2Params& p, const Launch& L, hipStream_t st);

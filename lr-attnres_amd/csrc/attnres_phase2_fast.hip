@@ -1,11 +1,14 @@
 // Phase 2, fast path for 16-bit rows that one wave covers exactly: D = 64
 // lanes x CB columns x one VB-byte vector (256 / 768 with 8-byte vectors,
 // 512 / 1024 with 16-byte ones).  Base keys (rms-norm of the scaled partial
-// block, scored against the query) with the addcmul merge and no output norm
+// block, scored against the query) with the addcmul merge
 // (reference: attention_residual_phase2, attnres_ops.py:3964-4035); LR keys
-// (r <= 256) with either merge and the optional output norm (reference:
-// lrid_attention_residual_phase2[_torch], attnres_ops.py:4075-4160).  Other
-// forms run the general kernels in attnres_phase2.hip.
+// (r <= 256) with either merge (reference:
+// lrid_attention_residual_phase2[_torch], attnres_ops.py:4075-4160); both with
+// or without the output norm.  Other forms run the general kernels in
+// attnres_phase2.hip.  Base keys with the output norm, D = 768, 16384 tokens,
+// bf16: forward 20.4 us in the general kernels, 16.1 here (4.7 TB/s); backward
+// 49 and 33.7 (3.7 TB/s; 123 registers, 4 waves per SIMD, bound by VALU work).
 //
 // The arithmetic and every rounding point are those of the general one-wave
 // kernels (the eager op's step-by-step roundings); only the instruction forms
@@ -13,7 +16,7 @@
 // work (phase 2 moves only 3 rows forward and 5 backward per token):
 //   * rows stay packed in the dtype; a rounding that feeds a packed consumer is
 //     one v_cvt_pk for two elements,
-//   * sums of dtype-rounded products (the logit <rnd(key), q> as the eager op
+//   * base keys without the output norm: sums of dtype-rounded products (the logit <rnd(key), q> as the eager op
 //     forms it, <g, rnd(p - it)>) add the packed products with one v_dot2
 //     against (1, 1); <p, p> is one v_dot2,
 //   * the query gradient adds rnd(dlb * key) from packed products with one
@@ -52,6 +55,53 @@ __device__ __forceinline__ void unpack2(uint32_t w, float& lo, float& hi) {
   hi = t[1];
 }
 
+// Sums over the row in the general kernels' order (per column, fp32 adds in
+// element order, then one wave sum per column added in column order), so the
+// per-token results are bit-identical to theirs.
+template <int CB>
+__device__ __forceinline__ float p2lr_row_sum(const float (&x)[CB]) {
+  float t = 0.f;
+#pragma unroll
+  for (int c = 0; c < CB; ++c) t += wave_sum(x[c]);
+  return t;
+}
+
+// The base kernels' row sums over packed words: with the output norm (SEQ) in
+// that order, without it two elements per v_dot2.
+template <class DT, int CB, bool SEQ>
+struct P2Sum {
+  float s[SEQ ? CB : 1];
+  __device__ __forceinline__ P2Sum() {
+#pragma unroll
+    for (int c = 0; c < (SEQ ? CB : 1); ++c) s[c] = 0.f;
+  }
+  __device__ __forceinline__ void add(int c, uint32_t x) {  // the two elements
+    if constexpr (SEQ) {
+      float a, b;
+      unpack2<DT>(x, a, b);
+      s[c] += a;
+      s[c] += b;
+    } else {
+      s[0] = dot2<DT>(x, one_pair<DT>(), s[0]);
+    }
+  }
+  __device__ __forceinline__ void add(int c, uint32_t x, uint32_t y) {  // their products
+    if constexpr (SEQ) {
+      float a, b, d, e;
+      unpack2<DT>(x, a, b);
+      unpack2<DT>(y, d, e);
+      s[c] += a * d;
+      s[c] += b * e;
+    } else {
+      s[0] = dot2<DT>(x, y, s[0]);
+    }
+  }
+  __device__ __forceinline__ float total() const {
+    if constexpr (SEQ) return p2lr_row_sum<CB>(s);
+    else return wave_sum(s[0]);
+  }
+};
+
 // The recomputed forward state of one token: scaled partial block p (packed,
 // dtype-rounded), rnd(p * inv) (packed, key norm), inv, sigmoid and its
 // dtype-rounded value.
@@ -63,13 +113,13 @@ struct P2Fast {
   float inv, sg, prob;
 };
 
-template <class DT, int VB, int CB, bool KN>
+template <class DT, int VB, int CB, bool KN, bool NM>
 __device__ __forceinline__ void p2fast_forward_state(const Phase2Params& p, const Raw<DT, VB / 2> (&pvr)[CB],
                                                      const float (&q)[CB][VB / 2], float vs, float bias, float lse,
                                                      P2Fast<DT, VB, CB, KN>& st) {
   constexpr int W = VB / 4;
   // p = rnd(pv * vs), packed; <p, p>
-  float ss = 0.f;
+  P2Sum<DT, CB, NM> ss;
 #pragma unroll
   for (int c = 0; c < CB; ++c)
 #pragma unroll
@@ -77,12 +127,12 @@ __device__ __forceinline__ void p2fast_forward_state(const Phase2Params& p, cons
       float a, b;
       unpack2<DT>(pvr[c].w[i], a, b);
       st.pw[c][i] = pack2<DT>(a * vs, b * vs);
-      if constexpr (KN) ss = dot2<DT>(st.pw[c][i], st.pw[c][i], ss);
+      if constexpr (KN) ss.add(c, st.pw[c][i], st.pw[c][i]);
     }
   st.inv = 1.f;
-  if constexpr (KN) st.inv = 1.0f / sqrtf(wave_sum(ss) / (float)p.D + p.eps);
+  if constexpr (KN) st.inv = 1.0f / sqrtf(ss.total() / (float)p.D + p.eps);
   // logit = rnd(sum_e rnd(key_e * q_e)), key = rnd(p * inv) (or p)
-  float t = 0.f;
+  P2Sum<DT, CB, NM> t;
 #pragma unroll
   for (int c = 0; c < CB; ++c)
 #pragma unroll
@@ -97,9 +147,9 @@ __device__ __forceinline__ void p2fast_forward_state(const Phase2Params& p, cons
         st.kw[c][i] = st.pw[c][i];
         unpack2<DT>(st.pw[c][i], k0, k1);
       }
-      t = dot2<DT>(pack2<DT>(k0 * q[c][2 * i], k1 * q[c][2 * i + 1]), one_pair<DT>(), t);
+      t.add(c, pack2<DT>(k0 * q[c][2 * i], k1 * q[c][2 * i + 1]));
     }
-  const float logit = DT::rnd(wave_sum(t));
+  const float logit = DT::rnd(t.total());
   const float x = (logit + bias) - lse;
   st.sg = 1.0f / (1.0f + expf(-x));
   st.prob = DT::rnd(st.sg);
@@ -123,7 +173,16 @@ __device__ __forceinline__ void p2fast_query(const Raw<DT, VB / 2> (&qr)[CB], fl
 
 }  // namespace
 
-template <class DT, int VB, int CB, bool KN>
+// addcmul merge of two elements: rnd(a + rnd(b - a) * w), a = interblock output, b = p
+template <class DT>
+__device__ __forceinline__ uint32_t p2fast_merge(uint32_t it, uint32_t pw, float w) {
+  float a0, a1, b0, b1, d0, d1;
+  unpack2<DT>(it, a0, a1);
+  unpack2<DT>(pw, b0, b1);
+  unpack2<DT>(pack2<DT>(b0 - a0, b1 - a1), d0, d1);
+  return pack2<DT>(a0 + d0 * w, a1 + d1 * w);
+}
+template <class DT, int VB, int CB, bool KN, bool NM>  // NM: output norm
 __global__ void __launch_bounds__(256) phase2_fwd_fast_kernel(const Phase2Params p) {
   using S = typename DT::S;
   constexpr int E = VB / 2;
@@ -148,28 +207,34 @@ __global__ void __launch_bounds__(256) phase2_fwd_fast_kernel(const Phase2Params
     float q[CB][E];
     p2fast_query<DT, VB, CB>(qr, q);
     P2Fast<DT, VB, CB, KN> st;
-    p2fast_forward_state<DT, VB, CB, KN>(p, pvr, q, vs, bias, p.lse[tok], st);
+    p2fast_forward_state<DT, VB, CB, KN, NM>(p, pvr, q, vs, bias, p.lse[tok], st);
     const float w = st.prob;
+    uint32_t ow[CB][W];
+    P2Sum<DT, CB, NM> ss;
+#pragma unroll
+    for (int c = 0; c < CB; ++c)
+#pragma unroll
+      for (int i = 0; i < W; ++i) {
+        ow[c][i] = p2fast_merge<DT>(itr[c].w[i], st.pw[c][i], w);
+        if constexpr (NM) ss.add(c, ow[c][i], ow[c][i]);
+      }
+    const float inv = NM ? 1.0f / sqrtf(ss.total() / (float)p.D + p.eps) : 1.f;
     S* op = (S*)p.out + tok * (int64_t)p.D;
 #pragma unroll
     for (int c = 0; c < CB; ++c) {
       float o[E];
 #pragma unroll
       for (int i = 0; i < W; ++i) {
-        // addcmul merge: rnd(a + rnd(b - a) * w), a = interblock output, b = p
-        float a0, a1, b0, b1, d0, d1;
-        unpack2<DT>(itr[c].w[i], a0, a1);
-        unpack2<DT>(st.pw[c][i], b0, b1);
-        unpack2<DT>(pack2<DT>(b0 - a0, b1 - a1), d0, d1);
-        o[2 * i] = a0 + d0 * w;
-        o[2 * i + 1] = a1 + d1 * w;
+        unpack2<DT>(ow[c][i], o[2 * i], o[2 * i + 1]);
+        o[2 * i] *= inv;  // the store rounds (exact when inv = 1)
+        o[2 * i + 1] *= inv;
       }
       store_vec<DT, E, true>(op + (c * kWave + lane) * E, o);
     }
   }
 }
 
-template <class DT, int VB, int CB, bool KN>
+template <class DT, int VB, int CB, bool KN, bool NM>  // NM: output norm
 __global__ void __launch_bounds__(256) phase2_bwd_fast_kernel(const Phase2Params p) {
   using S = typename DT::S;
   constexpr int E = VB / 2;
@@ -215,13 +280,39 @@ __global__ void __launch_bounds__(256) phase2_bwd_fast_kernel(const Phase2Params
       }
     }
     P2Fast<DT, VB, CB, KN> st;
-    p2fast_forward_state<DT, VB, CB, KN>(p, pvr, q, vs, bias, p.lse[tok], st);
+    p2fast_forward_state<DT, VB, CB, KN, NM>(p, pvr, q, vs, bias, p.lse[tok], st);
     const float w = st.prob;
+
+    // ---- the upstream gradient through the output norm, the merge worked out
+    // again: rnd(inv g - out inv^3 <g, out> / D)
+    if constexpr (NM) {
+      uint32_t ow[CB][W];
+      P2Sum<DT, CB, NM> oo, go;
+#pragma unroll
+      for (int c = 0; c < CB; ++c)
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+          ow[c][i] = p2fast_merge<DT>(itr[c].w[i], st.pw[c][i], w);
+          oo.add(c, ow[c][i], ow[c][i]);
+          go.add(c, gr[c].w[i], ow[c][i]);
+        }
+      const float inv = 1.0f / sqrtf(oo.total() / (float)D + p.eps);
+      const float k3 = inv * inv * inv * (go.total() / (float)D);
+#pragma unroll
+      for (int c = 0; c < CB; ++c)
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+          float g0, g1, o0, o1;
+          unpack2<DT>(gr[c].w[i], g0, g1);
+          unpack2<DT>(ow[c][i], o0, o1);
+          gr[c].w[i] = pack2<DT>(inv * g0 - o0 * k3, inv * g1 - o1 * k3);
+        }
+    }
 
     // ---- merge backward: d inter stored; d p (merge part) kept packed in gr;
     // dprob = rnd(sum_e rnd(g * rnd(p - it)))
     S* dip = (S*)p.dinter + tok * (int64_t)D;
-    float t = 0.f;
+    P2Sum<DT, CB, NM> t;
 #pragma unroll
     for (int c = 0; c < CB; ++c) {
       float di[E];
@@ -234,7 +325,7 @@ __global__ void __launch_bounds__(256) phase2_bwd_fast_kernel(const Phase2Params
         const uint32_t diff = pack2<DT>(b0 - a0, b1 - a1);
         float f0, f1;
         unpack2<DT>(diff, f0, f1);
-        t = dot2<DT>(pack2<DT>(g0 * f0, g1 * f1), one_pair<DT>(), t);
+        t.add(c, pack2<DT>(g0 * f0, g1 * f1));
         // d p (merge part) = rnd(g w), d inter = rnd(g - rnd(g w))
         const uint32_t dpm = pack2<DT>(g0 * w, g1 * w);
         float m0, m1;
@@ -245,7 +336,7 @@ __global__ void __launch_bounds__(256) phase2_bwd_fast_kernel(const Phase2Params
       }
       store_vec<DT, E, true>(dip + (c * kWave + lane) * E, di);
     }
-    const float dprob = DT::rnd(wave_sum(t));
+    const float dprob = DT::rnd(t.total());
     const float dx = dprob * (1.0f - st.sg) * st.sg;
     if (lane == 0) {
       p.dlse[tok] = -dx;
@@ -256,7 +347,7 @@ __global__ void __launch_bounds__(256) phase2_bwd_fast_kernel(const Phase2Params
     // ---- key backward: dq += rnd(dlb * key); <rnd(dlb q), p> for the rms-norm chain
     float k3 = 0.f;
     {
-      float m = 0.f;
+      P2Sum<DT, CB, NM> m;
 #pragma unroll
       for (int c = 0; c < CB; ++c)
 #pragma unroll
@@ -266,9 +357,9 @@ __global__ void __launch_bounds__(256) phase2_bwd_fast_kernel(const Phase2Params
           const uint32_t pr = pack2<DT>(dlb * k0, dlb * k1);
           dq[c][2 * i] = dot2<DT>(pr, e_lo, dq[c][2 * i]);
           dq[c][2 * i + 1] = dot2<DT>(pr, e_hi, dq[c][2 * i + 1]);
-          if constexpr (KN) m = dot2<DT>(pack2<DT>(dlb * q[c][2 * i], dlb * q[c][2 * i + 1]), st.pw[c][i], m);
+          if constexpr (KN) m.add(c, pack2<DT>(dlb * q[c][2 * i], dlb * q[c][2 * i + 1]), st.pw[c][i]);
         }
-      if constexpr (KN) k3 = st.inv * st.inv * st.inv * (wave_sum(m) / (float)D);
+      if constexpr (KN) k3 = st.inv * st.inv * st.inv * (m.total() / (float)D);
     }
     // ---- d p = rnd(rnd(dpm + dpk) * vs), dpk = rnd(inv * rnd(dlb q) - p * k3) (or rnd(dlb q))
     S* dpvp = (S*)p.dpv + tok * (int64_t)D;
@@ -350,17 +441,6 @@ __device__ __forceinline__ uint32_t p2lr_merge2(uint32_t aw, uint32_t bw, float 
     unpack2<DT>(pack2<DT>(b0 - a0, b1 - a1), d0, d1);
     return pack2<DT>(a0 + d0 * w, a1 + d1 * w);
   }
-}
-
-// Sums over the row in the general kernels' order (per column, fp32 adds in
-// element order, then one wave sum per column added in column order), so the
-// per-token results are bit-identical to theirs.
-template <int CB>
-__device__ __forceinline__ float p2lr_row_sum(const float (&x)[CB]) {
-  float t = 0.f;
-#pragma unroll
-  for (int c = 0; c < CB; ++c) t += wave_sum(x[c]);
-  return t;
 }
 
 // Recomputed forward state of one LR token: p = rnd(pv vs) packed, the key
@@ -833,8 +913,13 @@ namespace {
 template <class DT, int VB, int CB, bool KN>
 hipError_t p2fast_launch(bool bwd, const Phase2Params& p, const Launch& L, hipStream_t st) {
   const dim3 g(L.grid), b(kP2FastWaves * kWave);
-  if (bwd) hipLaunchKernelGGL((phase2_bwd_fast_kernel<DT, VB, CB, KN>), g, b, L.lds, st, p);
-  else hipLaunchKernelGGL((phase2_fwd_fast_kernel<DT, VB, CB, KN>), g, b, 0, st, p);
+  if (p.norm_out) {
+    if (bwd) hipLaunchKernelGGL((phase2_bwd_fast_kernel<DT, VB, CB, KN, true>), g, b, L.lds, st, p);
+    else hipLaunchKernelGGL((phase2_fwd_fast_kernel<DT, VB, CB, KN, true>), g, b, 0, st, p);
+  } else {
+    if (bwd) hipLaunchKernelGGL((phase2_bwd_fast_kernel<DT, VB, CB, KN, false>), g, b, L.lds, st, p);
+    else hipLaunchKernelGGL((phase2_fwd_fast_kernel<DT, VB, CB, KN, false>), g, b, 0, st, p);
+  }
   return hipGetLastError();
 }
 

@@ -2350,8 +2350,8 @@ bool value_keys_ok(const attnres_value_key_desc* d, int rank) {
 
 // Token parts per source for dW: at most two workgroups (of two waves per SIMD) per
 // CU over the column groups and sources, parts of at least 256 tokens.  17 sources
-// of D = 2048, 3 / 4 / 5 / 7 parts: 389 / 439 / 374 / 358 us, but 10 / 12 / 15 / 20
-// for the reduction; 9 sources of D = 768, 18 / 20 / 25 / 35: 29 / 34 / 30 / 33.
+// of D = 2048, 3 / 5 / 7 parts: 269 / 281 / 273 us and 10 / 17 / 22 for the
+// reduction; 9 sources of D = 768, 18 / 25 / 35: 26 / 28 / 29 and 9 / 12 / 14.
 int value_keys_parts(const attnres_value_key_desc* d) {
   const int64_t groups = (int64_t)((d->dim + 255) / 256) * d->n_src;
   const int64_t want = groups < 512 ? 512 / groups : 1, most = (d->n_tok + 255) / 256;

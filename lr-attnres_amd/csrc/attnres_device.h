@@ -448,9 +448,11 @@ __device__ __forceinline__ void wave_sync() {
 // wave-uniform.  The compiler does not order LDS reads after these loads:
 // read the row back only after wait_staged() (vmcnt(0): every vector-memory
 // operation of the wave has completed, these loads included).
+// NT: the non-temporal policy, for rows read once.
+template <bool NT = false>
 __device__ __forceinline__ void stage16(const void* src, void* lds_row) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                   (__attribute__((address_space(3))) void*)lds_row, 16, 0, 0);
+                                   (__attribute__((address_space(3))) void*)lds_row, 16, 0, NT ? 2 : 0);
 }
 __device__ __forceinline__ void wait_staged() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 

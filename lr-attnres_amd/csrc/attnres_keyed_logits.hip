@@ -6,7 +6,8 @@
 //   logits[q, s, t] = rnd(<queries[q], key[s, t]>)
 // The second half -- softmax over the sources, lse and the mix -- is exactly
 // phase 1 from these logits (attnres_phase1_forward), so the op composes the
-// two.  Backward, as the eager op's autograd:
+// two, for what the one-pass kernels of attnres_phase1_bank.hip do not take.
+// Backward, as the eager op's autograd:
 //   dkey = rnd(sum_q dl[q] queries[q]),  dv = rnd(inv (dkey - v inv mr)),
 //   mr = <dkey, v> inv / D  (key_norm; else dv = dkey),
 //   dqueries[q] = rnd(sum_{s,t} dl[q, s, t] key[s, t]).

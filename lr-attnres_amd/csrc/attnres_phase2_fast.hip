@@ -16,9 +16,9 @@
 // work (phase 2 moves only 3 rows forward and 5 backward per token):
 //   * rows stay packed in the dtype; a rounding that feeds a packed consumer is
 //     one v_cvt_pk for two elements,
-//   * base keys without the output norm: sums of dtype-rounded products (the logit <rnd(key), q> as the eager op
-//     forms it, <g, rnd(p - it)>) add the packed products with one v_dot2
-//     against (1, 1); <p, p> is one v_dot2,
+//   * base keys without the output norm: sums of dtype-rounded products (the
+//     logit <rnd(key), q> as the eager op forms it, <g, rnd(p - it)>) add the
+//     packed products with one v_dot2 against (1, 1); <p, p> is one v_dot2,
 //   * the query gradient adds rnd(dlb * key) from packed products with one
 //     v_dot2 against (1, 0) / (0, 1) per element.
 #include "attnres_device.h"

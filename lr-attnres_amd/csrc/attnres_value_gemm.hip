@@ -1,6 +1,5 @@
-// Value-derived LR keys with their projection on the matrix cores (config with
-// lrid_key_from_value and lrid_key_value_norm: LRIDSourceKeyProjection,
-// model.py:391-428):
+// Value-derived LR keys with their projection on the matrix cores
+// (LRIDSourceKeyProjection with its value norm, model.py:391-428):
 //   keys[s] = rnd(rnd(inv v[s]) W^T),  inv = 1 / sqrt(<v, v> / D + eps)
 //   dv[s]   = rnd(inv (gk W) - v inv^2 <gk, key> / D)
 //   dW      = rnd(sum_{s, t} rnd(inv gk)^T v)
@@ -25,15 +24,15 @@
 //            permuted so that a lane's two tiles are 8 consecutive columns of one
 //            row; B = 32 gradient rows, held throughout.
 //   dW       C = dW: k runs over tokens, so both operands are rows transposed:
-//            a lane loads 8 rows of a column pair (and of rank / 32 gradient
-//            columns) and pairs their halves with v_perm.  A wave holds all
-//            rank x 64 sums; workgroups split the tokens, and a second kernel adds
-//            their partial sums in a fixed order.
+//            a lane reads 8 rows of a column pair (and of rank / 32 gradient
+//            columns) from LDS and pairs their halves with v_perm.  A wave holds
+//            all rank x 64 sums; workgroups split the tokens, and a second kernel
+//            adds their partial sums in a fixed order.
 //
 // Measured with 17 sources of 16384 rows, D = 2048, rank 128, bf16 (one MI355X):
 // forward 388 us (was 357 for the norm and 287 for the GEMM), dv 585 (350 for the
-// GEMM and 591 for the norm's backward), dW 390 with its reduction 10 and the
-// gradient rows' preparation 38 (703 and 50 for stacking them): 1.40 ms of kernels
+// GEMM and 591 for the norm's backward), dW 262 with its reduction 10 and the
+// gradient rows' preparation 38 (703 and 50 for stacking them): 1.29 ms of kernels
 // against 2.34.  dv is at 78% of a copy's rate; the forward at the last-level
 // cache's for its second reading.
 #include "attnres_device.h"
@@ -305,20 +304,34 @@ __global__ void __launch_bounds__(256) value_keys_dv_kernel(const ValueKeysParam
   }
 }
 
-// partial dW of workgroup (column group x, token part y): tokens [t0, t1) of one source
+// partial dW of workgroup (column group x, token part y): tokens [t0, t1) of one source.
+// Stages of 32 rows x 256 columns and their gradient rows go straight from memory to
+// LDS (16 bytes a lane), two stages ahead of the one in use: 4.5 TB/s of rows, where
+// loads of a lane's own column pair into registers (4 bytes of a row a lane, 16 a
+// step, all that fit in flight) reached 2.9 (17 sources of 16384 rows, D = 2048, rank
+// 128: 262 us against 390; one source, D = 1024, rank 64: 10.8 against 16.7; cached
+// instead of streaming rows: 269).
+constexpr int kDwTok = 32, kDwStages = 3;
+constexpr int kDwRow = 512;  // bytes of a row in a stage
+template <int RT>
+constexpr int dw_stage_bytes() { return kDwTok * (kDwRow + 64 * RT); }
+
 template <int RT>
 __global__ void __launch_bounds__(256) value_keys_dw_kernel(const ValueKeysParams p) {
   using S = typename DT::S;
   constexpr int R = 32 * RT, GW = RT == 1 ? 1 : RT / 2;  // words of a lane's gradient columns (RT == 1: half of one)
-  const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+  constexpr int GI = RT == 4 ? 2 : 1;                    // a wave's gradient pieces of 1 KB (RT == 1: waves 2, 3 as 0, 1)
+  constexpr int kLoads = 4 + GI, kStage = dw_stage_bytes<RT>();
+  __shared__ __align__(16) char s_dw[kDwStages * kStage];  // [stages][rows' 256 columns | their gradient rows]
+  const int lane = threadIdx.x & 63, wave = uniform_i32(threadIdx.x / 64);
   const int l32 = lane & 31, h = lane >> 5;
   const int s = blockIdx.y / p.parts, part = blockIdx.y - s * p.parts, D = p.D;
   const int cb = (blockIdx.x * 4 + wave) * 64;
-  if (cb >= D) return;
   const int64_t per = (p.n_tok + p.parts - 1) / p.parts;
   const int64_t t0 = part * per, t1 = t0 + per < p.n_tok ? t0 + per : p.n_tok;
-  const char* vp = (const char*)((const S*)p.val[s] + cb + 2 * l32);
-  const char* gp = (const char*)((const S*)p.gs + (int64_t)s * p.n_tok * R + RT * l32);
+  const int col = min((int)blockIdx.x * 256 + 8 * l32, D - 8);  // the last group may be short: any column in its place
+  const char* vp = (const char*)((const S*)p.val[s] + col);
+  const char* gp = (const char*)((const S*)p.gs + (int64_t)s * p.n_tok * R);
   const int64_t vst = (int64_t)p.vstride[s] * 2;
 
   vk_f16 acc[RT][2];
@@ -328,31 +341,56 @@ __global__ void __launch_bounds__(256) value_keys_dw_kernel(const ValueKeysParam
     for (int T = 0; T < 2; ++T)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[t][T][i] = 0.f;
-  // two steps of 16 rows in flight: a buffer is loaded again as soon as its step
-  // has paired its words (one step ahead alone: 431 us against 405)
-  uint32_t va[8], ga[8][GW], vb[8], gb[8][GW];
-  // rows t + 8 h + j of this lane's columns (clamped to the last row of the part)
-  auto load = [&](int64_t t, uint32_t (&v)[8], uint32_t (&g)[8][GW]) {
+  // stage k: rows t = t0 + 32 k ... (past the part's end: its last row)
+  const int64_t v_lane = (8 * wave + h) * vst;
+  auto load = [&](int k, char* to) {
+    const int64_t t = t0 + (int64_t)k * kDwTok;
+    const bool whole = t + kDwTok <= t1;  // wave-uniform
+    const char* vt = vp + t * vst + v_lane;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const char* src = vt + 2 * q * vst;
+      if (!whole) {
+        const int64_t r = t + 8 * wave + 2 * q + h;
+        src = vp + (r < t1 ? r : t1 - 1) * vst;
+      }
+      stage16<true>(src, to + (8 * wave + 2 * q) * kDwRow);
+    }
+#pragma unroll
+    for (int i = 0; i < GI; ++i) {
+      const int piece = RT == 1 ? (wave & 1) : wave * GI + i, at = piece * 1024 + lane * 16;
+      const char* src = gp + t * (2 * R) + at;
+      if (!whole) {
+        const int64_t r = t + at / (2 * R);
+        src = gp + (r < t1 ? r : t1 - 1) * (2 * R) + at % (2 * R);
+      }
+      stage16(src, to + kDwTok * kDwRow + piece * 1024);
+    }
+  };
+  const int v_at = 8 * h * kDwRow + wave * 128 + 4 * l32, g_at = kDwTok * kDwRow + 8 * h * (2 * R) + 2 * RT * l32;
+  // 16 rows of a stage: row 8 h + j of this lane's columns
+  auto step = [&](const char* from, int64_t t, int row0) {
+    uint32_t v[8], g[8][GW];
+    const char* vl = from + v_at;
+    const char* gl = from + g_at;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int64_t r = t + 8 * h + j, rc = r < t1 ? r : t1 - 1;
-      v[j] = __builtin_nontemporal_load((const uint32_t*)(vp + rc * vst));
+      v[j] = *(const uint32_t*)(vl + (row0 + j) * kDwRow);
+      const char* gr = gl + (row0 + j) * (2 * R);
       if constexpr (RT == 4) {
-        const u32x2 x = *(const u32x2*)(gp + rc * R * 2);
+        const u32x2 x = *(const u32x2*)gr;
         g[j][0] = x.x;
         g[j][GW - 1] = x.y;
       } else if constexpr (RT == 2) {
-        g[j][0] = *(const uint32_t*)(gp + rc * R * 2);
+        g[j][0] = *(const uint32_t*)gr;
       } else {
-        g[j][0] = *(const uint16_t*)(gp + rc * R * 2);
+        g[j][0] = *(const uint16_t*)gr;
       }
     }
-  };
-  auto step = [&](int64_t t, uint32_t (&v)[8], uint32_t (&g)[8][GW]) {
-    if (t + 16 > t1) {  // wave-uniform: rows past the part's end count as zero
+    if (t + row0 + 16 > t1) {  // wave-uniform: rows past the part's end count as zero
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const bool ok = t + 8 * h + j < t1;
+        const bool ok = t + row0 + 8 * h + j < t1;
         v[j] = ok ? v[j] : 0u;
 #pragma unroll
         for (int i = 0; i < GW; ++i) g[j][i] = ok ? g[j][i] : 0u;
@@ -367,20 +405,28 @@ __global__ void __launch_bounds__(256) value_keys_dw_kernel(const ValueKeysParam
       for (int r = 0; r < RT; ++r)
         a[r][q] = (r & 1) ? hi_pair(g[2 * q][r / 2], g[2 * q + 1][r / 2]) : lo_pair(g[2 * q][r / 2], g[2 * q + 1][r / 2]);
     }
-    load(t + 32 < t1 ? t + 32 : t1 - 1, v, g);
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int T = 0; T < 2; ++T) acc[r][T] = vk_mfma(a[r], b[T], acc[r][T]);
   };
-  if (t0 < t1) {
-    load(t0, va, ga);
-    load(t0 + 16 < t1 ? t0 + 16 : t1 - 1, vb, gb);
-    for (int64_t t = t0; t < t1; t += 32) {
-      step(t, va, ga);
-      if (t + 16 < t1) step(t + 16, vb, gb);
-    }
+  const int n = t0 < t1 ? (int)((t1 - t0 + kDwTok - 1) / kDwTok) : 0;
+  for (int k = 0; k < kDwStages - 1 && k < n; ++k) load(k, s_dw + k * kStage);
+  int buf = 0;
+  for (int k = 0; k < n; ++k) {
+    // this wave's part of stage k has arrived (the next stage's loads may still run) ...
+    if (k + 1 < n) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kLoads * (kDwStages - 2)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();  // ... every wave's has, and none reads stage k - 1 any more
+    asm volatile("" ::: "memory");
+    const int ahead = buf == 0 ? kDwStages - 1 : buf - 1;
+    if (k + kDwStages - 1 < n) load(k + kDwStages - 1, s_dw + ahead * kStage);
+    const int64_t t = t0 + (int64_t)k * kDwTok;
+    step(s_dw + buf * kStage, t, 0);
+    step(s_dw + buf * kStage, t, 16);
+    buf = buf + 1 == kDwStages ? 0 : buf + 1;
   }
+  if (cb >= D) return;
   float* out = p.partials + (int64_t)blockIdx.y * R * D + cb + 2 * l32;
 #pragma unroll
   for (int r = 0; r < RT; ++r)

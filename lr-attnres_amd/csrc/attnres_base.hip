@@ -433,31 +433,20 @@ __global__ void __launch_bounds__(1024) reduce_partials_kernel(const ReduceParam
 
 // ============================================================== launchers
 // Workgroups of at most 256 threads may use up to 256 VGPRs per lane (the rows
-// of 16 sources stay resident without spilling); ONLY256 instantiates just
-// that bound, for layouts that always run one wave per token.
-template <class DT, int E, int CB, int NMAX, bool ONLY256 = false>
+// of 16 sources stay resident without spilling).
+template <class DT, int E, int CB, int NMAX>
 static hipError_t base_fwd_t(const ReadParams& p, const Launch& L, hipStream_t st) {
-  if (ONLY256 || L.wpt * kWave <= 256)
+  if (L.wpt * kWave <= 256)
     hipLaunchKernelGGL((base_fwd_kernel<DT, E, CB, NMAX, 256>), dim3(L.grid), dim3(L.wpt * kWave), L.lds, st, p);
-  else if constexpr (!ONLY256)
+  else
     hipLaunchKernelGGL((base_fwd_kernel<DT, E, CB, NMAX, 1024>), dim3(L.grid), dim3(L.wpt * kWave), L.lds, st, p);
   return hipGetLastError();
 }
 // Resident path (N <= 16): vector path keeps two columns per lane.  More
 // sources take the streaming kernels, which read each value row twice.
-// 16-bit rows of 256 or 768 elements use 8-byte vectors in one or three
-// columns, so that every lane of the wave holds part of the row (16-byte
-// vectors would leave half of the last column's lanes idle).
 template <class DT>
 static hipError_t base_fwd_dt(const ReadParams& p, const Launch& L, hipStream_t st) {
   constexpr int EV = 16 / sizeof(typename DT::S);
-  if constexpr (sizeof(typename DT::S) == 2) {
-    if (L.vec && L.vb == 8) {
-      if (L.wpt == 1 && p.ncols == 1)
-        return L.nmax == 8 ? base_fwd_t<DT, EV / 2, 1, 8, true>(p, L, st) : base_fwd_t<DT, EV / 2, 1, 16, true>(p, L, st);
-      return L.nmax == 8 ? base_fwd_t<DT, EV / 2, 3, 8, true>(p, L, st) : base_fwd_t<DT, EV / 2, 3, 16, true>(p, L, st);
-    }
-  }
   if (L.vec) {
     switch (L.nmax) {
       case 8: return base_fwd_t<DT, EV, 2, 8>(p, L, st);

@@ -328,28 +328,20 @@ __global__ void __launch_bounds__(1024) base_bwd_stream_kernel(const ReadBwdPara
 }
 
 // ============================================================== launchers
-template <class DT, int E, int CB, int NMAX, bool ONLY256 = false>
+template <class DT, int E, int CB, int NMAX>
 static hipError_t base_bwd_t(const ReadBwdParams& p, const Launch& L, hipStream_t st) {
   const int threads = L.wpt * kWave * L.teams;
-  if (ONLY256 || threads <= 256)
+  if (threads <= 256)
     hipLaunchKernelGGL((base_bwd_kernel<DT, E, CB, NMAX, 256>), dim3(L.grid), dim3(threads), L.lds, st, p);
-  else if constexpr (!ONLY256)
+  else
     hipLaunchKernelGGL((base_bwd_kernel<DT, E, CB, NMAX, 1024>), dim3(L.grid), dim3(threads), L.lds, st, p);
   return hipGetLastError();
 }
 
-// Resident path (N <= 16), 8-byte rows and streaming beyond 16 sources, as
-// in the forward.
+// Resident path (N <= 16) and streaming beyond 16 sources, as in the forward.
 template <class DT>
 static hipError_t base_bwd_dt(const ReadBwdParams& p, const Launch& L, hipStream_t st) {
   constexpr int EV = 16 / sizeof(typename DT::S);
-  if constexpr (sizeof(typename DT::S) == 2) {
-    if (L.vec && L.vb == 8) {
-      if (L.wpt == 1 && p.f.ncols == 1)
-        return L.nmax == 8 ? base_bwd_t<DT, EV / 2, 1, 8, true>(p, L, st) : base_bwd_t<DT, EV / 2, 1, 16, true>(p, L, st);
-      return L.nmax == 8 ? base_bwd_t<DT, EV / 2, 3, 8, true>(p, L, st) : base_bwd_t<DT, EV / 2, 3, 16, true>(p, L, st);
-    }
-  }
   if (L.vec) {
     switch (L.nmax) {
       case 8: return base_bwd_t<DT, EV, 2, 8>(p, L, st);

@@ -11,9 +11,10 @@ fallback and no dispatch switch.  Tensors that are not on a ROCm GPU, or a
 missing library, raise ``RuntimeError``.  ``force_triton`` is accepted for
 signature compatibility and has no effect (the HIP path is the only path).
 
-Autograd goes through ``torch.library.custom_op`` (``attnres_hip::read`` /
-``attnres_hip::read_backward``), with fake implementations for
-``torch.compile``.  The forward saves the fp32 softmax weights
+Eager calls go through autograd nodes, those of the reads and phases in C++
+(``_attnres_torch.so``), the others in Python; while ``torch.compile`` traces,
+through ``torch.library.custom_op`` (``attnres_hip::read`` /
+``attnres_hip::read_backward``, ...) with fake implementations.  The forward saves the fp32 softmax weights
 ``[B*T, H, N]``; the backward recomputes nothing from the keys except the key
 norm, and reduces cross-token gradients (static query, per-site gate, bias)
 deterministically.

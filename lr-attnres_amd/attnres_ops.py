@@ -458,7 +458,7 @@ def attention_residual_read(values, query: Tensor, key_norm: bool, force_triton:
     if nat:
         ok, bias = _native_bias(source_counts, source_logit_biases, values)
         out = nat.read(values, None, query, None, None, bias, None, 1, 1.0, bool(key_norm), bool(normalize_output),
-                       _hip.GATE_NONE) if ok else None
+                       _hip.GATE_NONE, False) if ok else None
         if out is not None:
             return out
     srcs = _sources(values)
@@ -558,7 +558,7 @@ def lrid_attention_residual_read(values, keys, query: Tensor, num_heads: int, lo
         ok, bias = _native_bias(source_counts, source_logit_biases, values)
         q = (None, query) if query.dim() == 4 else (query, None)
         out = nat.read(values, keys, *q, None, bias, static_keys, num_heads, float(logit_scale), bool(key_norm),
-                       bool(normalize_output), _hip.GATE_NONE) if ok else None
+                       bool(normalize_output), _hip.GATE_NONE, True) if ok else None
         if out is not None:
             return out
     vs, ks, H, D, R, k0_dtype = _lr_common(values, keys, num_heads, "lrid_attention_residual_read")
@@ -611,7 +611,7 @@ def lrid_attention_residual_read_gated(values, keys, static_query: Optional[Tens
         ok, bias = _native_bias(source_counts, source_logit_biases, values)
         out = nat.read(values, keys, static_query, dynamic_query, gate, bias, static_keys, num_heads,
                        float(logit_scale), bool(key_norm), bool(normalize_output),
-                       _GATE_ACTS[gate_activation] if gate is not None else _hip.GATE_NONE) if ok else None
+                       _GATE_ACTS[gate_activation] if gate is not None else _hip.GATE_NONE, False) if ok else None
         if out is not None:
             return out
     vs, ks, H, D, R, _ = _lr_common(values, keys, num_heads, "lrid_attention_residual_read_gated")

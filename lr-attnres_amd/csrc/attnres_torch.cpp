@@ -327,10 +327,11 @@ struct ReadFn : torch::autograd::Function<ReadFn> {
   }
 };
 
-// keys None: the base read.  query [H, R/H] or [D]; query_dyn [B, T, R] or [B, T, H, R/H]; gate [H] or [B, T, H]
+// keys None: the base read.  query [H, R/H] or [D]; query_dyn [B, T, H, R/H] or, unless by_heads, any [B, T, ...] of R
+// elements a token; gate [H] or [B, T, H]
 py::object attn_read(const py::object& values, const py::object& keys, const py::object& query, const py::object& query_dyn,
                 const py::object& gate, const py::object& bias, const py::object& static_keys, int64_t heads,
-                double scale, bool key_norm, bool normalize_output, int64_t gate_act) {
+                double scale, bool key_norm, bool normalize_output, int64_t gate_act, bool by_heads) {
   variable_list flat, ks;
   if (!plain_mode() || !unpack_list(values, &flat)) return py::none();
   const int64_t n = (int64_t)flat.size();
@@ -364,6 +365,7 @@ py::object attn_read(const py::object& values, const py::object& keys, const py:
   if (o[1].defined()) {
     if (!m->lr || !dense(o[1], dt, dev, B * T * R) || o[1].size(0) != B || o[1].dim() < 3 || o[1].size(1) != T)
       return py::none();
+    if (by_heads && (o[1].dim() != 4 || o[1].size(2) != heads)) return py::none();
     if (o[1].dim() != 3) o[1] = o[1].reshape({B, T, R});
   }
   if (o[2].defined()) {

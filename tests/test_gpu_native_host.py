@@ -152,6 +152,18 @@ def test_calls_it_leaves_to_python():
         assert str(e1.value) == str(e2.value)
 
 
+@pytest.mark.parametrize("shape", [(2, 4, 8, 2), (2, 4, 1, 16), (2, 4, 16, 1), (4, 2, 2, 8), (1, 8, 2, 8)])
+def test_a_per_token_query_of_another_shape_is_refused(shape):
+    """[B, T, H, R/H] is [2, 4, 2, 8] here: as many elements in another order or for other heads are an error."""
+    v, k = [_r(2, 4, 64) for _ in range(3)], [_r(2, 4, 16) for _ in range(3)]
+    call = lambda: ops.lrid_attention_residual_read(v, k, _r(*shape), 2, 0.25, True)  # noqa: E731
+    with pytest.raises(RuntimeError, match="per-token query must be") as e1:
+        call()
+    with _python_route(), pytest.raises(RuntimeError) as e2:
+        call()
+    assert str(e1.value) == str(e2.value)
+
+
 def _block(D=256, R=32, Q=3, S=3, T=5):
     return lambda: dict(v=[_r(2, T, D) for _ in range(S)], lg=[_r(Q, 2, T, dtype=torch.float32) for _ in range(S)],
                         y=[_r(2, T, D + R + 8) for _ in range(Q)], bank=_r(4, R), qs=_r(Q, D, std=0.1), pv=_r(2, T, D),

@@ -145,9 +145,10 @@ void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 float* fptr(const Tensor& t) { return t.defined() ? t.data_ptr<float>() : nullptr; }
 
 // the first node of an error when gradients of these gradients are asked for
-// (the backwards are not differentiable)
-variable_list once(variable_list grads) {
-  if (!at::GradMode::is_enabled()) return grads;
+// (the backwards are not differentiable); plain gradients when no incoming one
+// requires a gradient, as torch's once_differentiable returns them
+variable_list once(variable_list grads, const variable_list& incoming) {
+  if (!any_grad(incoming)) return grads;
   variable_list have;
   for (const Tensor& g : grads)
     if (g.defined()) have.push_back(g);
@@ -323,7 +324,7 @@ struct ReadFn : torch::autograd::Function<ReadFn> {
     // inputs that need no gradient get none (the kernels write all of them in one pass)
     for (size_t i = 0; i < n_in; ++i)
       if (ctx->needs_input_grad(i)) res[1 + i] = d[i];
-    return once(std::move(res));
+    return once(std::move(res), grads);
   }
 };
 
@@ -475,7 +476,7 @@ struct Phase1Fn : torch::autograd::Function<Phase1Fn> {
         if (ctx->needs_input_grad(n + i)) res[n + i] = dvs[i];
       }
     }
-    return once(std::move(res));
+    return once(std::move(res), grads);
   }
 };
 
@@ -589,7 +590,7 @@ struct BankFn : torch::autograd::Function<BankFn> {
       for (int i = 0; i < n; ++i)
         if (ctx->needs_input_grad(1 + i)) res[2 + i] = dvs[i];
     }
-    return once(std::move(res));
+    return once(std::move(res), grads);
   }
 };
 
@@ -712,7 +713,7 @@ struct Phase2Fn : torch::autograd::Function<Phase2Fn> {
       for (size_t i = 0; i < s.size(); ++i)
         if (ctx->needs_input_grad(i)) res[1 + i] = all[i];
     }
-    return once(std::move(res));
+    return once(std::move(res), grads);
   }
 };
 
@@ -862,7 +863,7 @@ struct AccumReadFn : torch::autograd::Function<AccumReadFn> {
       for (size_t i = 0; i < n_in; ++i)
         if (ctx->needs_input_grad(i)) res[1 + i] = all[i];
     }
-    return once(std::move(res));
+    return once(std::move(res), grads);
   }
 };
 
@@ -981,7 +982,7 @@ struct AccumFn : torch::autograd::Function<AccumFn> {
         if (ctx->needs_input_grad(2) && gk.defined()) res[3] = gk;
       }
     }
-    return once(std::move(res));
+    return once(std::move(res), grads);
   }
 };
 

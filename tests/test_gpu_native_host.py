@@ -208,6 +208,31 @@ def test_one_backward_only():
         g.float().sum().backward()
 
 
+@pytest.mark.parametrize("name", ["read", "phase1", "bank", "phase2", "accum", "accum_read"])
+def test_create_graph_under_a_constant_upstream_gradient(name):
+    """create_graph with an upstream gradient that needs none: the gradients are constants of the next backward, on
+    both routes (an incoming gradient that needs one makes them an error: test_one_backward_only)."""
+    i = _block()()
+    call = {"read": lambda: ops.attention_residual_read(i["v"], i["q"], True),
+            "phase1": lambda: ops.lrid_block_phase1(i["v"], i["lg"])[0][1],
+            "bank": lambda: ops.attention_residual_phase1(i["v"], i["qs"], True)[0],
+            "phase2": lambda: ops.attention_residual_phase2(i["v"][0], i["q"], i["inter"], i["lse"], True),
+            "accum": lambda: ops.lrid_block_accumulate(i["y"][0], i["pv"], i["pk"], 256, 32, complete=True)[0],
+            "accum_read": lambda: ops.lrid_block_accumulate_read(i["y"][0], i["pv"], i["pk"], i["bank"], i["inter"],
+                                                                 i["lse"], 256, 32, 0.2, query_row=1)[2]}[name]
+    x = i["y"][0] if name.startswith("accum") else i["v"][0]
+
+    def second():
+        out = call()
+        (g,) = torch.autograd.grad(out, [x], torch.ones_like(out), create_graph=True)
+        assert not g.requires_grad
+        return torch.autograd.grad((g.float() * x.float()).sum(), [x])[0]
+
+    got = second()
+    with _python_route():
+        assert torch.equal(got, second())
+
+
 def test_saved_tensor_hooks_and_in_place_changes():
     torch.manual_seed(1)
     v, q = [_r(1, 3, 64) for _ in range(3)], _r(64, std=0.2)

@@ -346,9 +346,11 @@ _BOUND = {name: getattr(_hip, name) for name in (
 
 def _native(fwd: str, bwd: str):
     global _NATIVE
+    if _compiling():  # (before the load below: torch.compile cannot trace it)
+        return None
     if _NATIVE is None:
         _NATIVE = _hip.native() if torch.cuda.is_available() else False
-    if _NATIVE is False or _compiling():
+    if _NATIVE is False:
         return None
     return _NATIVE if getattr(_hip, fwd) is _BOUND[fwd] and getattr(_hip, bwd) is _BOUND[bwd] else None
 

@@ -9,6 +9,10 @@ the library-op path (schemas, fake shapes, autograd registration) without any
 code generation; results must equal the eager calls exactly.
 """
 
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -85,3 +89,24 @@ def test_compiled_phase_schedule_matches_eager():
         return ops.attention_residual_phase2(t[S + 1], t[S + 2], outs[0], lse[0], True) + outs[1]
 
     _compare(fn, [*vals, logits, partial, q], up)
+
+
+_FIRST = """
+import torch
+import attnres_ops as ops
+torch.manual_seed(0)
+v = [torch.randn(2, 8, 256, device="cuda", dtype=torch.bfloat16, requires_grad=True) for _ in range(3)]
+q = torch.randn(256, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+fn = lambda: ops.attention_residual_read(v, q, True)
+got = torch.compile(fn, backend="aot_eager", fullgraph=True)()
+got = [got.detach(), *torch.autograd.grad(got, [*v, q], torch.ones_like(got))]
+want = fn()
+want = [want.detach(), *torch.autograd.grad(want, [*v, q], torch.ones_like(want))]
+assert all(torch.equal(a, b) for a, b in zip(got, want))
+"""
+
+
+def test_the_first_call_of_a_process_may_be_a_compiled_one():
+    env = dict(os.environ, PYTHONPATH=os.path.dirname(os.path.abspath(ops.__file__)))
+    r = subprocess.run([sys.executable, "-c", _FIRST], env=env, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-3000:]

@@ -356,16 +356,23 @@ def _native(fwd: str, bwd: str):
 
 
 def _native_bias(source_counts, source_logit_biases, values):
-    """(whether the native call can take the logit bias, the bias)."""
+    """(whether the native call can take the logit bias, the bias).  Raises nothing: what the Python
+    checks would refuse, or pass over for a single source, is left to them."""
     if source_counts is None and source_logit_biases is None:
         return True, None
-    if isinstance(source_logit_biases, Tensor):
-        return source_counts is None, source_logit_biases
-    n = len(values)
-    given = source_logit_biases if source_counts is None else source_counts
-    if n == 0 or not isinstance(given, (list, tuple)) or len(given) != n or not isinstance(values, (list, tuple)):
+    if source_counts is not None and source_logit_biases is not None:
         return False, None
-    if not all(type(x) in (float, int) for x in given) or not values[0].is_cuda:
+    if isinstance(source_logit_biases, Tensor):
+        return True, source_logit_biases
+    given = source_logit_biases if source_counts is None else source_counts
+    if not isinstance(values, (list, tuple)) or not isinstance(given, (list, tuple)):
+        return False, None
+    n = len(values)
+    if n < 2 or len(given) != n or not all(type(x) in (float, int) for x in given):
+        return False, None
+    if source_counts is not None and any(c <= 0 for c in given):
+        return False, None
+    if not isinstance(values[0], Tensor) or not values[0].is_cuda:
         return False, None
     return True, _source_logit_bias(source_counts, source_logit_biases, n, values[0].device)
 

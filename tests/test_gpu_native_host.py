@@ -164,6 +164,29 @@ def test_a_per_token_query_of_another_shape_is_refused(shape):
     assert str(e1.value) == str(e2.value)
 
 
+def test_biases_and_queries_the_python_checks_judge():
+    """A single source passes over its counts, sources may come from a generator, what was refused stays refused."""
+    v, k = [_r(2, 4, 64) for _ in range(3)], [_r(2, 4, 16) for _ in range(3)]
+    qb, q, qd = _r(64), _r(1, 16), _r(2, 4, 1, 16)
+    base, lr, gated = ops.attention_residual_read, ops.lrid_attention_residual_read, ops.lrid_attention_residual_read_gated
+    both = dict(source_counts=[1, 2, 3], source_logit_biases=[0.0, 0.1, 0.2])
+    for call in (lambda: base(v[:1], qb, True, source_counts=[0]), lambda: lr(v[:1], k[:1], q, 1, 0.25, True, source_counts=[-1]),
+                 lambda: gated(v[:1], k[:1], q, qd, None, 1, 0.25, True, source_counts=[0]),
+                 lambda: base(v[:1], qb, True, source_counts=[1], source_logit_biases=[0.0]),
+                 lambda: base((t for t in v), qb, True, source_counts=[1, 2, 3]),
+                 lambda: lr((t for t in v), (t for t in k), q, 1, 0.25, True, source_logit_biases=[0.1, 0.2, 0.3])):
+        got = call()
+        with _python_route():
+            assert torch.equal(got, call())
+    for call in (lambda: base(v, qb, True, source_counts=[1, 0, 2]),
+                 lambda: lr(v, k, q, 1, 0.25, True, **both), lambda: base(v, qb, True, source_counts=[1, 2])):
+        with pytest.raises((RuntimeError, AttributeError)) as e1:
+            call()
+        with _python_route(), pytest.raises((RuntimeError, AttributeError)) as e2:
+            call()
+        assert e1.type is e2.type and str(e1.value) == str(e2.value)
+
+
 def _block(D=256, R=32, Q=3, S=3, T=5):
     return lambda: dict(v=[_r(2, T, D) for _ in range(S)], lg=[_r(Q, 2, T, dtype=torch.float32) for _ in range(S)],
                         y=[_r(2, T, D + R + 8) for _ in range(Q)], bank=_r(4, R), qs=_r(Q, D, std=0.1), pv=_r(2, T, D),

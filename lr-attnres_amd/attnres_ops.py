@@ -616,7 +616,7 @@ def lrid_attention_residual_read_gated(values, keys, static_query: Optional[Tens
     in ``lrid_attention_residual_read`` (config 4's [N, 128] static source key).
     """
     nat = _native("forward", "backward")
-    if nat and type(num_heads) is int and gate_activation in _GATE_ACTS:
+    if nat and dynamic_query is not None and type(num_heads) is int and gate_activation in _GATE_ACTS:
         ok, bias = _native_bias(source_counts, source_logit_biases, values)
         out = nat.read(values, keys, static_query, dynamic_query, gate, bias, static_keys, num_heads,
                        float(logit_scale), bool(key_norm), bool(normalize_output),

@@ -178,7 +178,7 @@ def test_biases_and_queries_the_python_checks_judge():
         got = call()
         with _python_route():
             assert torch.equal(got, call())
-    for call in (lambda: base(v, qb, True, source_counts=[1, 0, 2]),
+    for call in (lambda: gated(v, k, q, None, None, 1, 0.25, True), lambda: base(v, qb, True, source_counts=[1, 0, 2]),
                  lambda: lr(v, k, q, 1, 0.25, True, **both), lambda: base(v, qb, True, source_counts=[1, 2])):
         with pytest.raises((RuntimeError, AttributeError)) as e1:
             call()

@@ -355,11 +355,17 @@ def native():
 
 
 def available() -> bool:
+    """Whether the calls can run: a GPU, the library and the host extension, which every eager call (none that is
+    traced) asks for."""
     try:
         load()
-    except (OSError, RuntimeError):
+        if not torch.cuda.is_available():
+            return False
+        if not torch.compiler.is_compiling():
+            native()
+    except (OSError, RuntimeError, ImportError):
         return False
-    return torch.cuda.is_available()
+    return True
 
 
 def _ptr(t):

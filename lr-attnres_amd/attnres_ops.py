@@ -54,7 +54,7 @@ _GATE_ACTS = {"linear": _hip.GATE_LINEAR, "sigmoid": _hip.GATE_SIGMOID}
 
 
 def is_fused_attnres_available() -> bool:
-    """True when the HIP library loads and a ROCm GPU is visible (reference: attnres_ops.py:123-124)."""
+    """True when the HIP library and the host extension load and a ROCm GPU is visible (reference: attnres_ops.py:123-124)."""
     return _hip.available()
 
 

@@ -417,7 +417,7 @@ class _ReadFn(torch.autograd.Function):
         n_v, n_k, has, heads, logit_scale, key_norm, normalize_output, mode, gate_act, gate_per_token, _ = ctx.meta
         saved = ctx.saved_tensors  # (checks that no input was modified in place)
         query, query_dyn, gate, bias, static_keys = _unflatten_opt(has, saved[n_v + n_k:-3])
-        pre, w, inv = saved[-3:]
+        pre, w, inv = (t.contiguous() for t in saved[-3:])  # (a saved-tensor hook may give back another layout)
         B, T, D = ctx.shape
         dev = saved[0].device
         want = ctx.needs_input_grad
@@ -1009,6 +1009,11 @@ class _Phase1BankFn(torch.autograd.Function):
         queries, logits, inv, *values = ctx.saved_tensors
         if grad_out is None and grad_lse is None:
             return (None, None, *([None] * len(values)))
+        # (a saved-tensor hook may give back another layout or alignment)
+        queries, logits, inv = queries.contiguous(), logits.contiguous(), inv.contiguous()
+        values = [v if v.stride(-1) == 1 else v.contiguous() for v in values]
+        if not _hip.phase1_bank_fits(_hip.KeyedLogits(values, queries, ctx.key_norm)):
+            queries, *values = [t.clone(memory_format=torch.contiguous_format) for t in (queries, *values)]
         v0 = values[0]
         Q, n, D = queries.size(0), v0.size(0), v0.size(1)
         grad_out = v0.new_zeros((Q, n, D)) if grad_out is None else grad_out.contiguous()
@@ -1523,6 +1528,11 @@ class _ValueKeyGemmFn(torch.autograd.Function):
         n, (B, T, _), R = len(values), values[0].shape, weight.size(0)
         if all(g is None for g in grad_keys):
             return (None,) * (1 + n)
+        # (a saved-tensor hook may give back another layout or alignment)
+        weight, keys, inv = weight.contiguous(), keys.contiguous(), inv.contiguous()
+        values = [_hip.as_rows(v) for v in values]
+        if keys.data_ptr() % 16 or not _hip.value_keys_fits(_hip.ValueKey(values), weight):
+            weight, keys, *values = [t.clone(memory_format=torch.contiguous_format) for t in (weight, keys, *values)]
         gk = [None if g is None else g.reshape(B * T, R).contiguous() for g in grad_keys]
         gk = [g.clone() if g is not None and g.data_ptr() % 16 else g for g in gk]  # (views into larger gradients)
         want = ctx.needs_input_grad

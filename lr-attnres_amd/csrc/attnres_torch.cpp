@@ -13,7 +13,8 @@
 //
 // Nothing of a call outlives it but the autograd node's saved tensors: the
 // backward builds its descriptor from the tensors it unpacks (so saved-tensor
-// hooks and in-place checks hold), on the stream current then.
+// hooks hold, whatever layout they give back, and in-place checks), on the
+// stream current then.
 #include <dlfcn.h>
 
 #include <limits>
@@ -164,6 +165,17 @@ variable_list once(variable_list grads, const variable_list& incoming) {
   return grads;
 }
 
+// Saved tensors as the kernels address them: a saved-tensor hook may give a tensor back in another layout.  Those that
+// may be strided rows (rows(i)) are copied unless they are; the others are made dense.
+template <class F>
+void lay_out(variable_list* s, F rows) {
+  for (size_t i = 0; i < s->size(); ++i) {
+    Tensor& t = (*s)[i];
+    if (t.defined() && !t.is_contiguous() && !(rows(i) && t.dim() == 3 && row_stride(t) >= 0)) t = t.contiguous();
+  }
+}
+void copy_dense(Tensor* t) { *t = t->clone(at::MemoryFormat::Contiguous); }
+
 struct Pointers {
   const void* p[ATTNRES_MAX_SOURCES];
   int64_t s[ATTNRES_MAX_SOURCES];
@@ -282,6 +294,8 @@ struct ReadFn : torch::autograd::Function<ReadFn> {
     variable_list d;
     {
       at::NoGradGuard no_grad;
+      const size_t n_rows = (m->lr ? 2 : 1) * (size_t)m->n;
+      lay_out(&s, [&](size_t i) { return i < n_rows; });
       ReadCall c(*m, s.data());
       c10::DeviceGuard guard(c.dev);
       const auto opt = s[0].options().requires_grad(false);
@@ -439,6 +453,7 @@ struct Phase1Fn : torch::autograd::Function<Phase1Fn> {
     variable_list res(s.size());
     {
       at::NoGradGuard no_grad;
+      lay_out(&s, [&](size_t i) { return i >= (size_t)n; });
       attnres_phase1_desc d;
       Pointers v;
       const void* lg[ATTNRES_MAX_SOURCES];
@@ -563,9 +578,14 @@ struct BankFn : torch::autograd::Function<BankFn> {
     if (!grads[0].defined() && !grads[1].defined()) return res;
     {
       at::NoGradGuard no_grad;
+      lay_out(&s, [&](size_t i) { return i > 0 && i <= (size_t)n; });
       attnres_keyed_logits_desc d;
       Pointers v;
       describe(*m, s.data(), n, &d, &v);
+      if (!lib.attnres_phase1_bank_fits(&d)) {  // (given back at another alignment)
+        for (int i = 0; i <= n; ++i) copy_dense(&s[i]);
+        describe(*m, s.data(), n, &d, &v);
+      }
       const Tensor& v0 = s[1];
       c10::DeviceGuard guard(v0.device());
       const auto opt = v0.options().requires_grad(false);
@@ -683,6 +703,7 @@ struct Phase2Fn : torch::autograd::Function<Phase2Fn> {
     {
       at::NoGradGuard no_grad;
       const bool lr = s.size() > 4;
+      lay_out(&s, [](size_t i) { return i < 2 || i == 4; });
       attnres_phase2_desc d;
       fill_merge(*m, s[0], lr ? s[4] : Tensor(), s[3], s[1], s[2], s[0].size(2), &d);
       const auto dev = s[0].device();
@@ -787,6 +808,11 @@ Tensor grad_rows(const Tensor& g, int64_t W, int64_t* stride) {
   return g.contiguous();
 }
 
+// rows of whole 16-byte vectors, as the fused kernels read them
+bool fused_rows(const Tensor& t) {
+  return ((uintptr_t)t.data_ptr() | (uintptr_t)(row_stride(t) * t.element_size())) % 16 == 0;
+}
+
 struct AccumReadFn : torch::autograd::Function<AccumReadFn> {
   // in: y [B, T, P], query bank [rows, R], inter [B, T, D], lse [B, T], and the old partial value and key
   static variable_list run(const MergeMeta& m, const variable_list& in, Tensor* kinv) {
@@ -825,6 +851,9 @@ struct AccumReadFn : torch::autograd::Function<AccumReadFn> {
     if (!grads[0].defined() && !grads[1].defined() && !grads[2].defined()) return res;
     {
       at::NoGradGuard no_grad;
+      lay_out(&s, [](size_t i) { return i == 2; });
+      for (size_t i : {(size_t)0, (size_t)2, n_in + 1})  // (given back at another alignment)
+        if (!fused_rows(s[i])) copy_dense(&s[i]);
       const Tensor &y = s[0], &query = s[1], &inter = s[2], &lse = s[3], &kinv = s[n_in], &value = s[n_in + 1],
                    &key = s[n_in + 2];
       const int64_t n = inter.size(0) * inter.size(1);
@@ -895,7 +924,7 @@ py::object accum_read(const py::object& projected, const py::object& partial_val
   if (es != 2 || (D != 256 && D != 512 && D != 768 && D != 1024) || R > 256) return py::none();
   int64_t st[1];
   if (!same_rows({it}, B, T, dt, dev, st) || it.size(2) != D || !dense(ls, at::kFloat, dev, B * T)) return py::none();
-  if (((uintptr_t)y.data_ptr() | (uintptr_t)it.data_ptr() | (y.size(2) * es) | (st[0] * es)) % 16) return py::none();
+  if (!fused_rows(y) || !fused_rows(it)) return py::none();
   if (q.dim() != 2 || q.size(1) != R || query_row < 0 || query_row >= q.size(0) || !dense(q, dt, dev, q.size(0) * R))
     return py::none();
   auto m = c10::make_intrusive<MergeMeta>();
@@ -963,6 +992,7 @@ struct AccumFn : torch::autograd::Function<AccumFn> {
     if (!grads[0].defined() && !grads[1].defined()) return res;
     {
       at::NoGradGuard no_grad;
+      lay_out(&s, [](size_t) { return false; });
       const Tensor& y = s[0];
       const int64_t n = y.size(0) * y.size(1);
       c10::DeviceGuard guard(y.device());

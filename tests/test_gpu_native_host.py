@@ -271,6 +271,65 @@ def test_saved_tensor_hooks_and_in_place_changes():
         out.float().sum().backward()
 
 
+def _swapped(t):
+    """The same values, the last two dimensions swapped in memory (or every second element of a row)."""
+    if t.dim() < 2:
+        out = t.new_empty((2 * t.numel(),))[::2].view(t.shape)
+    else:
+        out = t.new_empty((*t.shape[:-2], t.size(-1), t.size(-2))).transpose(-1, -2)
+    return out.copy_(t)
+
+
+def _shifted(t):
+    """The same values, one element into a buffer."""
+    return torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
+
+
+_HOOKED = {
+    "base": lambda i: ops.attention_residual_read(i["v"], i["q"], True, normalize_output=True),
+    "lr": lambda i: ops.lrid_attention_residual_read(i["v"], i["k"], i["qh"], 2, 0.25, True),
+    "gated": lambda i: ops.lrid_attention_residual_read_gated(i["v"], i["k"], i["qh"], i["qd"], i["gate"], 2, 0.25, True,
+                                                              static_keys=i["sk"]),
+    "phase1": lambda i: ops.lrid_block_phase1(i["v"], i["lg"]),
+    "bank": lambda i: ops.attention_residual_phase1(i["v"], i["qs"], True),
+    "phase2": lambda i: ops.attention_residual_phase2(i["pv"], i["q"], i["inter"], i["lse"], True),
+    "phase2_lr": lambda i: ops.lrid_attention_residual_phase2(i["pv"], i["pk"], i["bank"], i["inter"], i["lse"], 0.2, True,
+                                                              query_row=1),
+    "accum": lambda i: ops.lrid_block_accumulate(i["y"][0], i["pv"], i["pk"], 256, 32, complete=True, partial_scale=0.5),
+    "accum_read": lambda i: ops.lrid_block_accumulate_read(i["y"][0], i["pv"], i["pk"], i["bank"], i["inter"], i["lse"], 256,
+                                                           32, 0.2, query_row=1),
+    "value_keys": lambda i: ops.lrid_value_key_projection(i["v"], i["bank_w"]),
+}
+
+
+@pytest.mark.parametrize("route", [contextlib.nullcontext, _python_route])
+@pytest.mark.parametrize("name", list(_HOOKED))
+@pytest.mark.parametrize("unpack", [_swapped, _shifted])
+def test_saved_tensor_hooks_may_change_the_layout(unpack, name, route):
+    torch.manual_seed(5)
+    i = _block()()
+    i.update(k=[_r(2, 5, 32) for _ in range(3)], qh=_r(2, 16), qd=_r(2, 5, 2, 16), gate=_r(2, 5, 2), sk=_r(3, 32),
+             bank_w=_r(32, 256))
+    leaves = [t for t in _flat(list(i.values())) if t.requires_grad]
+    with route():
+        def grads():
+            outs = _flat(_HOOKED[name](i))
+            torch.manual_seed(6)
+            return torch.autograd.grad(outs, leaves, [torch.randn_like(o) for o in outs], allow_unused=True)
+
+        want = grads()
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            got = grads()
+    for a, b in zip(got, want):
+        assert (a is None) == (b is None)
+        if a is None:
+            continue
+        if unpack is _swapped:
+            assert torch.equal(a, b)
+        else:  # (kernels of another alignment may add in another order: an ulp of the largest element)
+            assert (a.float() - b.float()).abs().max() <= 2.0 ** -7 * max(1.0, b.float().abs().max().item())
+
+
 def test_transforms_and_modes_are_not_passed_by():
     v, q = [_r(1, 3, 64, grad=False) for _ in range(2)], _r(64, grad=False)
     with pytest.raises(Exception):

@@ -1724,8 +1724,10 @@ class _AccumReadFn(torch.autograd.Function):
         want = ctx.needs_input_grad  # (meta, y, pv, pk, query, inter, lse, bias, scale)
         d = ctx.desc
         g_out = torch.zeros_like(value) if g_out is None else g_out.contiguous()
-        if g_value is not None and (g_value.stride(-1) != 1 or g_value.stride(0) < dim):
-            g_value = g_value.contiguous()
+        if not _fused_rows(g_out):
+            g_out = g_out.clone()
+        if g_value is not None and (g_value.stride(-1) != 1 or g_value.stride(0) < dim or not _fused_rows(g_value)):
+            g_value = g_value.clone(memory_format=torch.contiguous_format)
         gk = g_key.contiguous() if g_key is not None else None
         dev = y.device
         with _device_ctx(dev):
@@ -1747,7 +1749,12 @@ def _accum_read_fits(y: Tensor, inter: Tensor, D: int, R: int, heads: int) -> bo
         return False
     if not 1 <= R <= 256 or R % heads != 0:
         return False
-    return all(t.data_ptr() % 16 == 0 and (t.stride(0) * t.element_size()) % 16 == 0 for t in (y, inter))
+    return all(_fused_rows(t) for t in (y, inter))
+
+
+def _fused_rows(t: Tensor) -> bool:
+    """Rows [n, W] of whole 16-byte vectors, as the fused kernels read them."""
+    return t.data_ptr() % 16 == 0 and (t.stride(0) * t.element_size()) % 16 == 0
 
 
 def lrid_block_accumulate_read(projected: Tensor, partial_value: Optional[Tensor], partial_key: Optional[Tensor],
@@ -1795,7 +1802,8 @@ def lrid_block_accumulate_read(projected: Tensor, partial_value: Optional[Tensor
     y = projected.reshape(B * T, P) if projected.numel() == B * T * P else None
     inter = _rows2d(interblock_output) if interblock_output.dtype == projected.dtype else None
     fused = (y is not None and inter is not None and y.stride(-1) == 1 and B * T > 0 and not _compiling()
-             and P >= D + R and _accum_read_fits(y, inter, D, R, int(num_heads)))
+             and P >= D + R and _accum_read_fits(y, inter, D, R, int(num_heads))
+             and (partial_value is None or partial_value.data_ptr() % 16 == 0 or not partial_value.is_contiguous()))
     if not fused:
         value, key = lrid_block_accumulate(projected, partial_value, partial_key, D, R, num_heads, key_norm)
         value, key = value.reshape(B, T, D), key.reshape(B, T, R)

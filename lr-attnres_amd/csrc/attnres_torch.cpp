@@ -863,10 +863,15 @@ struct AccumReadFn : torch::autograd::Function<AccumReadFn> {
       attnres_accum_read_desc d;
       fill_split(*m, y, m->has_partial ? s[4] : Tensor(), m->has_partial ? s[5] : Tensor(), false, 1.f, n, &d.accum);
       fill_merge(*m, value, key, query, inter, lse, m->D, &d.read);
-      const Tensor go = grads[2].defined() ? grads[2].contiguous() : at::zeros(value.sizes(), opt);
+      Tensor go = grads[2].defined() ? grads[2].contiguous() : at::zeros(value.sizes(), opt);
+      if (!fused_rows(go)) copy_dense(&go);
       int64_t gvs = m->D;
       Tensor gv, gk;
       if (grads[0].defined()) gv = grad_rows(grads[0], m->D, &gvs);
+      if (gv.defined() && !fused_rows(gv)) {
+        copy_dense(&gv);
+        gvs = m->D;
+      }
       if (grads[1].defined()) gk = grads[1].contiguous();
       Tensor gy = at::empty(y.sizes(), opt), di = at::empty(inter.sizes(), opt);
       Tensor dl = at::empty(lse.sizes(), opt.dtype(at::kFloat)), dq, dpk;
@@ -909,7 +914,7 @@ bool accum_inputs(const py::object& projected, const py::object& partial_value, 
   return true;
 }
 
-// the caller has checked that the fused kernels take the rows (_accum_read_fits)
+// the checks here decide whether the fused kernels take the rows (for the Python route: _accum_read_fits)
 py::object accum_read(const py::object& projected, const py::object& partial_value, const py::object& partial_key,
                       const py::object& bank, const py::object& inter, const py::object& lse, int64_t D, int64_t R,
                       double scale, int64_t heads, bool key_norm, bool merge_key_norm, int64_t merge,
@@ -924,7 +929,7 @@ py::object accum_read(const py::object& projected, const py::object& partial_val
   if (es != 2 || (D != 256 && D != 512 && D != 768 && D != 1024) || R > 256) return py::none();
   int64_t st[1];
   if (!same_rows({it}, B, T, dt, dev, st) || it.size(2) != D || !dense(ls, at::kFloat, dev, B * T)) return py::none();
-  if (!fused_rows(y) || !fused_rows(it)) return py::none();
+  if (!fused_rows(y) || !fused_rows(it) || (pv.defined() && !fused_rows(pv))) return py::none();
   if (q.dim() != 2 || q.size(1) != R || query_row < 0 || query_row >= q.size(0) || !dense(q, dt, dev, q.size(0) * R))
     return py::none();
   auto m = c10::make_intrusive<MergeMeta>();

@@ -233,3 +233,70 @@ def test_accumulate_read_empty_batch(fused_calls):
     o.sum().backward()
     assert float(lf[3].grad.abs().max()) == 0.0
     assert len(fused_calls) == 0
+
+
+@pytest.fixture(params=["native", "python"])
+def route_calls(request, monkeypatch):
+    """One of the two host routes, and its calls that reached the fused kernels (the tests above follow the Python one:
+    a replaced binding is called)."""
+    calls = []
+    if request.param == "python":
+        real = H.accum_read_forward
+        monkeypatch.setattr(ops, "_NATIVE", False)
+        monkeypatch.setattr(H, "accum_read_forward", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+        return calls
+    nat = H.native()
+
+    class Counting:
+        def __getattr__(self, name):
+            return getattr(nat, name)
+
+        def accum_read(self, *a):
+            res = nat.accum_read(*a)
+            calls.extend([1] if res is not None else [])
+            return res
+
+    monkeypatch.setattr(ops, "_NATIVE", Counting())
+    return calls
+
+
+def _equal_to_the_composition(ins, D, R, heads, key_norm, kw, go, gv, gk, place=lambda t, name: t):
+    names = ("y", "pv", "pk", "query", "inter", "lse")
+    res = []
+    for fused in (True, False):
+        lv = [place(t.detach().clone(), n).requires_grad_(True) if t is not None else None
+              for t, n in zip(_leaves(ins, DEV), names)]
+        out = _run(fused, lv, D, R, heads, key_norm, kw, place(go.to(DEV), "go"), place(gv.to(DEV), "gv"), gk.to(DEV))
+        res.append([*out, *[t.grad for t in lv if t is not None]])
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("D,R,P,heads,key_norm", CASES)
+@pytest.mark.parametrize("first", [False, True])
+def test_accumulate_read_on_both_routes(route_calls, D, R, P, heads, key_norm, first):
+    dtype = torch.bfloat16
+    g = gen(D + R + first)
+    ins = _inputs(g, 2, 37, D, R, D + P, dtype, first, 6)
+    kw = dict(lerp=True, normalize_output=True, logit_bias=0.37, partial_scale=3.0 ** -0.5, scale_key=not key_norm,
+              query_row=3)
+    _equal_to_the_composition(ins, D, R, heads, key_norm, kw, randn(g, (2, 37, D), dtype), randn(g, (2, 37, D), dtype),
+                              randn(g, (2, 37, R), dtype))
+    assert len(route_calls) == 1
+
+
+@pytest.mark.parametrize("which", ["y", "pv", "pk", "inter", "go", "gv"])
+def test_accumulate_read_of_misaligned_rows(route_calls, which):
+    """One tensor a single element into its buffer: inputs the fused kernels cannot read compose the two calls, upstream
+    gradients are copied."""
+    dtype, D, R = torch.bfloat16, 768, 64
+    g = gen(17)
+    ins = _inputs(g, 2, 9, D, R, D + R, dtype, False, 6)
+    kw = dict(lerp=False, normalize_output=True, logit_bias=0.37, partial_scale=0.5, scale_key=False, query_row=3)
+
+    def place(t, name):
+        return torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape) if name == which else t
+
+    _equal_to_the_composition(ins, D, R, 1, True, kw, randn(g, (2, 9, D), dtype), randn(g, (2, 9, D), dtype),
+                              randn(g, (2, 9, R), dtype), place)
+    assert len(route_calls) == (0 if which in ("y", "pv", "inter") else 1)

@@ -478,9 +478,11 @@ struct Phase1Fn : torch::autograd::Function<Phase1Fn> {
         }
       }
       void *dv[ATTNRES_MAX_SOURCES], *dl[ATTNRES_MAX_SOURCES];
-      variable_list dvs = at::empty({n, v0.size(0), v0.size(1), v0.size(2)}, opt).unbind(0);
+      // (an allocation per source: a source that later blocks read too keeps its gradient long after the others')
+      variable_list dvs(n);
       variable_list dls = at::empty({n, Q, v0.size(0), v0.size(1)}, opt.dtype(s[0].scalar_type())).unbind(0);
       for (int i = 0; i < n; ++i) {
+        dvs[i] = at::empty(v0.sizes(), opt);
         dv[i] = dvs[i].data_ptr();
         dl[i] = dls[i].data_ptr();
       }

@@ -231,6 +231,16 @@ def test_one_backward_only():
         g.float().sum().backward()
 
 
+@pytest.mark.parametrize("route", [contextlib.nullcontext, _python_route])
+def test_a_block_sources_gradient_outlives_the_others_alone(route):
+    """Phase 1's value gradients are allocations of their own: one that is kept does not hold the others' memory."""
+    i = _block(D=256, T=512)()
+    with route():
+        outs, _ = ops.lrid_block_phase1(i["v"], i["lg"])
+        g = torch.autograd.grad(outs, i["v"], [torch.ones_like(o) for o in outs])
+    assert len({t.untyped_storage().data_ptr() for t in g}) == len(g)
+
+
 @pytest.mark.parametrize("name", ["read", "phase1", "bank", "phase2", "accum", "accum_read"])
 def test_create_graph_under_a_constant_upstream_gradient(name):
     """create_graph with an upstream gradient that needs none: the gradients are constants of the next backward, on

@@ -768,7 +768,7 @@ extern "C" int attnres_read_backward(const attnres_read_desc* d, const attnres_r
     L.grid = (int)(need < full_groups ? need : full_groups);
   }
   hipStream_t st = (hipStream_t)stream;
-  int partials_layout = kPartRowMajor;  // fast LR: slot-major; fast base: tiled (slot-major for tiny inputs)
+  int partials_layout = kPartRowMajor;  // LR fast and split: slot-major; base fast and split: tiled where that fits
   BaseFastPlan bf;
   hipError_t err;
   const bool timed = timer_begin(st);
@@ -847,9 +847,13 @@ extern "C" int attnres_read_backward(const attnres_read_desc* d, const attnres_r
     L.wpt = sp.wpt;
     L.nmax = sp.nb;
     L.grid = (int)full_groups;  // d1024 N 9 / d640 N 7, 1024 / 1280 / 2048 workgroups: 160, 57 / 154, 51 / 149, 50 us
-    // (as the fast backward: tiles unless they would not fit the workspace)
+    // tiles, or whole rows where the padded tiles would not fit the workspace (a
+    // bias and at most 2048 tokens): these are written in runs, where slot-major
+    // sums cost a line per slot (bf16 d2048 N 5, output norm and bias, 128 / 512 /
+    // 2048 tokens: slot-major 15.6 / 35.5 / 132.6 us, rows 10.4 / 18.0 / 52.4;
+    // the step-by-step kernels 17.2 / 25.9 / 65.8)
     partials_layout =
-        (size_t)L.grid * part_stride(PL.n_part) <= (size_t)groups * PL.n_part ? kPartTiled : kPartSlotMajor;
+        (size_t)L.grid * part_stride(PL.n_part) <= (size_t)groups * PL.n_part ? kPartTiled : kPartRowMajor;
     bp.part_layout = partials_layout;
     err = launch_base_split_backward(d->dtype, bp, L, st);
   } else {

@@ -366,6 +366,22 @@ struct LrSplitPlan {
   int vb, wpt, nb, nh, np, kch, ki;
 };
 
+// The forward stays on the step-by-step kernels where every wave of a wide head
+// would score all N keys for itself over many registers of values, and the
+// tokens fill the chip without it: 16-bit heads of six or more waves (8-byte
+// vectors, beyond 32 sources) or of four with 41 to 52 sources, and fp32 rows
+// beyond 1024 with many sources of a short rank.  Step by step / split, us,
+// forward: bf16 one head, N 49, 2048 tokens of d2048 r 128 109 / 184, 16384 of
+// d1024 r 32 339 / 394; N 64, 1024 of d2048 r 32 91 / 75.  fp32, 4096 tokens: d1280
+// H 5 r 40 N 17 77 / 115, d1536 r 32 N 25 137 / 169, d2048 r 64 N 17 152 / 135.
+bool lr_split_forward_pays(const attnres_read_desc* d, int waves_per_head) {
+  const int N = d->n_src, D = d->dim, R = d->rank;
+  if (d->dtype == ATTNRES_DTYPE_F32)
+    return !(d->n_tok > 512 && D > 1024 && (R / d->heads <= 8 || (N > 16 && (R < 64 || (R <= 160 && D < 2048)))));
+  if (N <= 32) return true;
+  return !((waves_per_head >= 6 && d->n_tok > 1024) || (waves_per_head >= 4 && N > 40 && N <= 52 && d->n_tok > 2048));
+}
+
 bool lr_split_plan(const attnres_read_desc* d, const Plan& pl, bool backward, LrSplitPlan* f) {
   if (!pl.lr || !pl.vec || !pl.key_vec) return false;
   if (!d->query || d->query_dyn || d->gate || d->static_keys) return false;
@@ -377,6 +393,7 @@ bool lr_split_plan(const attnres_read_desc* d, const Plan& pl, bool backward, Lr
   if (es == 4 && N > 32) return false;
   const int E = f->vb / es, colw = kWaveSize * E;
   if (D > 2048 || D % E || dh % (16 * E) || H > 255) return false;
+  if (!backward && !lr_split_forward_pays(d, dh / colw)) return false;
   f->wpt = (D + colw - 1) / colw;
   f->nb = lr_split_slots(N);
   f->np = 2;

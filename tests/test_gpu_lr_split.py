@@ -41,6 +41,31 @@ def test_split_read_walks_tokens(norm):
     _lr_case(7400, torch.bfloat16, 1, 4099, 192, 3, 16, 1, 0.25, True, normalize_output=norm)
 
 
+@pytest.mark.parametrize("dtype,D,S,R,line", [(torch.float32, 1280, 17, 32, 512), (torch.float32, 1536, 3, 8, 512),
+                                              (torch.bfloat16, 1536, 33, 32, 1024), (torch.float16, 1024, 41, 16, 2048)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_split_read_forward_line(dtype, D, S, R, line, norm):
+    """One token past the line the forward runs step by step (the backward stays split): results and gradients are those
+    of the two parts, which take the split kernels, to the roundings of the order of fp32 sums: 16 of an fp32 ulp, or one
+    step of the 16-bit type (2^-8, 2^-11 relative) in every element at worst."""
+    import attnres_ops as ops
+
+    g = torch.Generator(device="cuda").manual_seed(7500 + D)
+    n, cut = line + 1, line // 2
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda").to(dtype)  # noqa: E731
+    vals, keys, q, up = [rn(1, n, D) for _ in range(S)], [rn(1, n, R) for _ in range(S)], rn(1, R), rn(1, n, D)
+
+    def run(a, b):
+        vs, ks = ([t[:, a:b].contiguous().requires_grad_(True) for t in x] for x in (vals, keys))
+        out = ops.lrid_attention_residual_read(vs, ks, q, 1, 0.25, True, normalize_output=norm)
+        return [out.detach(), *torch.autograd.grad(out, [*vs, *ks], up[:, a:b].contiguous())]
+
+    tol = {torch.float32: 2.0 ** -20, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for whole, x, y in zip(run(0, n), run(0, cut), run(cut, n)):
+        parts = torch.cat([x, y], 1).double()
+        assert float((whole.double() - parts).norm() / parts.norm()) <= tol
+
+
 def test_split_read_infinite_rows():
     """An infinity in a weighted source stays in its column; odd source counts pair the last row with zeros, not with itself."""
     import attnres_ops as ops

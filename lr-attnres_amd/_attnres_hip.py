@@ -1078,9 +1078,21 @@ def value_keys_fits(d: ValueKey, weight) -> bool:
             and bool(load().attnres_value_keys_fits(ctypes.byref(d.c), int(weight.size(0)))))
 
 
+def _few_value_key_rows(rows: int, D: int, R: int) -> bool:
+    """Rows (tokens of all sources) so few and so long that the norm and a library GEMM are the faster forward.  The
+    projection kernel walks a row twice in 64-column steps, a chain of 15 ns a column at rank 128 (9 at 32) that few
+    workgroups cannot hide; a second launch costs an eager caller about 23 us.  One source of 4096, rank 128, 64 tokens,
+    us, kernel against norm and GEMM: device 62 / 18, an eager call 61 / 51; 16384 tokens 195 / 311.  Of 2048, rank 128,
+    64 tokens: device 34 / 14, but an eager call 33 / 50."""
+    return R == 128 and D > 3072 and rows <= 4 * D
+
+
 def value_keys_forward(d: ValueKey, weight, for_backward: bool):
     """(keys [N, n_tok, R], inv_rms [N, n_tok] | None)."""
     R = weight.size(0)
+    if _few_value_key_rows(d.n_src * d.n_tok, d.D, R):
+        normed, inv = value_norm_forward(d, weight.device, weight.dtype)
+        return torch.mm(normed, weight.t()).view(d.n_src, d.n_tok, R), inv
     keys = torch.empty((d.n_src, d.n_tok, R), device=weight.device, dtype=weight.dtype)
     inv = torch.empty((d.n_src, d.n_tok), device=weight.device, dtype=torch.float32) if for_backward else None
     rc = load().attnres_value_keys_forward(ctypes.byref(d.c), _ptr(weight), R, _ptr(keys), _fptr(inv),

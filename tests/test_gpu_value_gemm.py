@@ -62,6 +62,20 @@ def test_token_counts(n_tok):
     _check(2, 1, n_tok, 256, 64)
 
 
+@pytest.mark.parametrize("D,R,line", [(4096, 128, 16384), (3136, 128, 12544)])
+def test_forward_line(D, R, line):
+    """Rows up to the line take the norm and the library GEMM, one more the projection kernel; same keys either way, to
+    the rounding of another order of fp32 sums (one bf16 step in every element at worst), with and without gradients."""
+    torch.manual_seed(D + R)
+    v = torch.randn((1, line + 1, D), device="cuda").to(BF)
+    w = (torch.randn((R, D), device="cuda") * D ** -0.5).to(BF)
+    with torch.no_grad():
+        (more,), (up_to,) = (ops.lrid_value_key_projection([v[:, :n]], w) for n in (line + 1, line))
+    _close(more[:, :line], up_to.double(), "keys", 2.0 ** -8)
+    (k,) = ops.lrid_value_key_projection([v[:, :line].requires_grad_(True)], w)
+    assert torch.equal(k.detach(), up_to)
+
+
 def test_one_source_many_parts():
     _check(1, 1, 5000, 512, 128)
 

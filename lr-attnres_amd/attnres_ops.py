@@ -1553,7 +1553,8 @@ def lrid_value_key_projection(values, weight: Tensor, value_norm: bool = True):
     each way (the normed rows never leave the registers); other forms rms-norm
     every source in one HIP pass (fp32, one rounding to the dtype) into one block,
     project all of them with a single library GEMM, and run the GEMMs for the
-    weight and input gradients and one HIP pass of the rms-norm backward.  ``values``: N x [B, T, D] (or [N, B, T, D]); ``weight`` [R, D]
+    weight and input gradients and one HIP pass of the rms-norm backward.
+    ``values``: N x [B, T, D] (or [N, B, T, D]); ``weight`` [R, D]
     (``nn.Linear(D, R).weight``).  Returns N keys [B, T, R] in the values' dtype.
     """
     vs = _sources(values)

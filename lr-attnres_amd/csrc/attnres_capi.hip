@@ -359,8 +359,10 @@ bool lr_fast_plan(const attnres_read_desc* d, const Plan& pl, bool backward, Fas
 // which holds four per lane.
 // Grids, us at 16384 tokens of d768 (N 13) / d1024 (N 13) / at 8192 of d1024 (N 25),
 // one head: forward 2048 / 4096 / 8192 / 16384 workgroups 92, 98, 107 / 86, 101,
-// 101 / 85, 99, 98 / 89, 98, 98; backward 1024 / 1536 / 2048 / 4096 150, 190,
-// 189 / 166, 190, 194 / 157, 204, 199 / 154, 192, 190.
+// 101 / 85, 99, 98 / 89, 98, 98.  Backward with its reduction, 1024 / 2048 / 4096
+// workgroups, 16384 tokens: d768 N 13 157 / 167 / 160, d1024 N 13 190 / 202 / 192,
+// N 25 352 / 365 / 351, d2048 N 9 257 / 250 / 244, d640 N 5 88 / 68 / 76, d768 N 4
+// 70 / 61 / 71: 4096, the workspace's rows, is never far from the best.
 constexpr int kLrSplitFwdGroups = 8192;
 struct LrSplitPlan {
   int vb, wpt, nb, nh, np, kch, ki;
@@ -492,7 +494,10 @@ bool base_fast_plan(const attnres_read_desc* d, const Plan& pl, BaseFastPlan* f)
 // sources fit the registers (d1024 N 9, output norm, 16384 tokens: 67 against
 // 71 us with 8-byte ones), else in 8-byte ones; the backward always in 8-byte
 // ones, at twice the waves and half the registers (the same read: 149 against
-// 161 us; N 25, 8192 tokens: 203 against 242).
+// 161 us; N 25, 8192 tokens: 203 against 242).  From 49 sources on the backward
+// spills (bf16 / fp16 at 52, 56, 60, 64 slots: 7 / 12, 23 / 40, 55 / 44, 84 / 86
+// registers) and still beats the streaming kernels: d1024, 8192 tokens, N 52 447
+// against 815 us, N 64 642 against 1063.
 struct BaseSplitPlan {
   int vb, wpt, nb;
 };
@@ -1752,7 +1757,7 @@ namespace {
 
 // Shapes of attnres_phase1_bank.hip: a wave per 256 columns with four elements
 // per lane, at most eight waves, 12 source and 12 site slots (the register
-// budget: 12 sources and 12 sites take 228 VGPRs in the backward).
+// budget: attnres_phase1_bank.hip).
 bool phase1_bank_plan(const attnres_keyed_logits_desc* d, Phase1BankParams* p, Launch* L) {
   if (d->n_tok <= 0 || d->n_src > kBankMaxSources || d->n_q > kBankMaxSites || d->dim > kBankMaxDim) return false;
   if (d->dim % 4) return false;
@@ -1781,10 +1786,15 @@ bool phase1_bank_plan(const attnres_keyed_logits_desc* d, Phase1BankParams* p, L
   return true;
 }
 
-// Workgroups: each loads the bank once and walks tokens.  Backward workgroups
-// also write one partial row of Q * D sums; one resident round of three waves
-// per SIMD is best (attnres_phase1_bank.hip).  Forward, 2048 / 4096 / 16384:
-// 78 / 65 / 66 us at 6 sources, 4 sites, D = 768, 16384 tokens.
+// Workgroups: each loads the bank once and walks tokens; backward ones also
+// write one partial row of Q * D sums.  One count for all shapes, chosen at 6
+// sources, 4 sites, D = 768, 16384 tokens, bf16 (forward 2048 / 4096 / 16384: 78 /
+// 65 / 66 us; backward with its reduction 512 / 1024 / 1280 / 1536 / 2048 / 4096:
+// 169 / 128 / 129 / 138 / 135 / 134).  It is not a resident round: that is 4 to 8
+// waves per SIMD by the slots, of ceil(D / 256) waves a workgroup.  So narrower
+// rows would take more workgroups and wider ones fewer: backward, D = 256, 512 /
+// 1280 / 2048 123 / 74 / 56 us; D = 2048 290 / 307 / 312; and 4096 tokens, which
+// 1280 does not divide, D = 768 1024 / 1280 41 / 49.
 constexpr int kBankFwdGroups = 4096;
 constexpr int kBankBwdGroups = 1280;
 int64_t bank_groups(int64_t n_tok, int64_t cap) { return n_tok < cap ? n_tok : cap; }

@@ -18,7 +18,11 @@
 // Layout: one workgroup per token at a time, a wave per 256 columns (four
 // elements per lane), so that S value rows, Q upstream rows, the bank (loop
 // invariant, in registers) and the backward's bank-gradient sums (Q x 4 per
-// lane, written once per workgroup) all fit.  Row sums are folded per wave
+// lane, written once per workgroup) fit: the backward at 2 sources and sites /
+// 6 and 4 / 12 and 12 takes 62 / 111 / 228 registers in bf16, 60 / 119 / 256 in
+// fp16 and 74 / 149 / 256 in fp32, where 12 and 12 spills 109 words (8 and 12
+// under 20), still four times faster than the two kernel families (d768, 4096
+// tokens, forward and backward: 440 us against 2363).  Row sums are folded per wave
 // (wave_sums) and added over the waves through LDS in a fixed order: two
 // barriers per token, the buffers alternating between tokens.  The (site,
 // source) pairs -- lane = q * np + s, np a power of two, 64 pairs at a time --
@@ -32,8 +36,7 @@
 // kernel families and 110 us of gradient adds before.  What is left is
 // instructions: about 760 vector and 280 scalar ones per token and wave in the
 // backward, against 910 slots in the token's bytes at the copy rate; loading a
-// token ahead changed nothing.  The backward's grid is one resident round
-// (1024 / 1280 / 1536 / 2560 workgroups: 130 / 118 / 126 / 125 us).
+// token ahead changed nothing.
 #include "attnres_device.h"
 #include "attnres_launch.h"
 #include "attnres_params.h"

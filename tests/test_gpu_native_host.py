@@ -342,10 +342,10 @@ def test_saved_tensor_hooks_may_change_the_layout(unpack, name, route):
 
 def test_transforms_and_modes_are_not_passed_by():
     v, q = [_r(1, 3, 64, grad=False) for _ in range(2)], _r(64, grad=False)
-    with pytest.raises(Exception):
+    with pytest.raises(RuntimeError, match="autograd.Function with functorch transforms"):
         torch.func.vmap(lambda a: ops.attention_residual_read([a, v[1]], q, True))(torch.stack([v[0], v[0]]))
     import torch.autograd.forward_ad as fwAD
-    with fwAD.dual_level(), pytest.raises(Exception):
+    with fwAD.dual_level(), pytest.raises(NotImplementedError, match="forward mode AD"):
         d = fwAD.make_dual(v[0], torch.ones_like(v[0]))
         ops.attention_residual_read([d, v[1].requires_grad_()], q, True)
 

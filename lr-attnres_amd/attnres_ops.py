@@ -1012,8 +1012,10 @@ class _Phase1BankFn(torch.autograd.Function):
         # (a saved-tensor hook may give back another layout or alignment)
         queries, logits, inv = queries.contiguous(), logits.contiguous(), inv.contiguous()
         values = [v if v.stride(-1) == 1 else v.contiguous() for v in values]
-        if not _hip.phase1_bank_fits(_hip.KeyedLogits(values, queries, ctx.key_norm)):
+        desc = _hip.KeyedLogits(values, queries, ctx.key_norm)
+        if not _hip.phase1_bank_fits(desc):
             queries, *values = [t.clone(memory_format=torch.contiguous_format) for t in (queries, *values)]
+            desc = _hip.KeyedLogits(values, queries, ctx.key_norm)
         v0 = values[0]
         Q, n, D = queries.size(0), v0.size(0), v0.size(1)
         grad_out = v0.new_zeros((Q, n, D)) if grad_out is None else grad_out.contiguous()
@@ -1022,8 +1024,7 @@ class _Phase1BankFn(torch.autograd.Function):
         grad_lse = grad_lse.float().contiguous() if grad_lse is not None else None
         want = ctx.needs_input_grad
         with _device_ctx(v0.device):
-            dvals, dq = _hip.phase1_bank_backward(_hip.KeyedLogits(values, queries, ctx.key_norm), v0.device, v0.dtype,
-                                                  grad_out, grad_lse, logits, inv, bool(want[1]))
+            dvals, dq = _hip.phase1_bank_backward(desc, v0.device, v0.dtype, grad_out, grad_lse, logits, inv, bool(want[1]))
         return (None, dq, *[d if want[2 + i] else None for i, d in enumerate(dvals)])
 
 
@@ -1531,14 +1532,15 @@ class _ValueKeyGemmFn(torch.autograd.Function):
         # (a saved-tensor hook may give back another layout or alignment)
         weight, keys, inv = weight.contiguous(), keys.contiguous(), inv.contiguous()
         values = [_hip.as_rows(v) for v in values]
-        if keys.data_ptr() % 16 or not _hip.value_keys_fits(_hip.ValueKey(values), weight):
+        desc = _hip.ValueKey(values)
+        if keys.data_ptr() % 16 or not _hip.value_keys_fits(desc, weight):
             weight, keys, *values = [t.clone(memory_format=torch.contiguous_format) for t in (weight, keys, *values)]
+            desc = _hip.ValueKey(values)
         gk = [None if g is None else g.reshape(B * T, R).contiguous() for g in grad_keys]
         gk = [g.clone() if g is not None and g.data_ptr() % 16 else g for g in gk]  # (views into larger gradients)
         want = ctx.needs_input_grad
         with _device_ctx(weight.device):
-            dvals, dw = _hip.value_keys_backward(_hip.ValueKey(values), weight, gk, keys, inv, any(want[1:]), want[0],
-                                                 (B, T))
+            dvals, dw = _hip.value_keys_backward(desc, weight, gk, keys, inv, any(want[1:]), want[0], (B, T))
         return (dw, *[dvals[i] if want[1 + i] else None for i in range(n)])
 
 

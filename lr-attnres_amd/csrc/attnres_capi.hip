@@ -507,6 +507,13 @@ bool base_split_plan(const attnres_read_desc* d, const Plan& pl, bool backward, 
   const int es = elem_size(d->dtype), N = d->n_src, D = d->dim;
   if (D > 2048 || (es == 4 && N > 32)) return false;
   f->vb = es == 4 || (!backward && D % 512 == 0 && N <= 32) ? 16 : 8;
+  // two or three rows in 8-byte vectors leave a token's waves mostly waiting for
+  // one another: the resident step-by-step forward then (us, that / this, bf16, 8192
+  // tokens, output norm: d768 N 2 16.7 / 19.4, d1800 N 2 36.6 / 50.9, N 3 44.5 / 50.9;
+  // but N 4 51.8 / 50.8, and 1024 tokens of d1472 N 2 8.5 / 8.3)
+  if (!backward && f->vb == 8 && d->n_tok >= 2048 && D > 512 &&
+      ((N <= 2 && (d->normalize_output || D > 1280)) || (N == 3 && d->normalize_output && D > 1280)))
+    return false;
   const int colw = kWaveSize * (f->vb / es);
   f->wpt = (D + colw - 1) / colw;
   f->nb = lr_split_slots(N);

@@ -62,6 +62,29 @@ def test_split_base_walks_tokens(norm):
     assert float((whole[-1].double() - total).norm() / total.norm()) < 10 * 2.0 ** -9
 
 
+@pytest.mark.parametrize("D,S,norm", [(640, 2, True), (1288, 2, False), (1288, 3, True)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_split_base_forward_line(dtype, D, S, norm):
+    """2048 tokens of two or three such rows run the resident forward (the backward stays split): results and gradients are
+    those of the halves, which take the split one, to the rounding of another order of fp32 sums, one step of the type in
+    every element at worst."""
+    import attnres_ops as ops
+
+    g = torch.Generator(device="cuda").manual_seed(8500 + D)
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda").to(dtype)  # noqa: E731
+    vals, q, up = [rn(1, 2048, D) for _ in range(S)], rn(D) * 0.03, rn(1, 2048, D)
+
+    def run(a, b):
+        vs = [v[:, a:b].contiguous().requires_grad_(True) for v in vals]
+        out = ops.attention_residual_read(vs, q, True, normalize_output=norm)
+        return [out.detach(), *torch.autograd.grad(out, vs, up[:, a:b].contiguous())]
+
+    tol = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for whole, x, y in zip(run(0, 2048), run(0, 1024), run(1024, 2048)):
+        parts = torch.cat([x, y], 1).double()
+        assert float((whole.double() - parts).norm() / parts.norm()) <= tol
+
+
 def test_split_base_infinite_rows():
     """An infinity in a source keeps out of the others: odd source counts pair the last row with zeros, not with itself."""
     import attnres_ops as ops

@@ -355,6 +355,9 @@ def _native(fwd: str, bwd: str):
     return _NATIVE if getattr(_hip, fwd) is _BOUND[fwd] and getattr(_hip, bwd) is _BOUND[bwd] else None
 
 
+_NUMBERS = frozenset((float, int))
+
+
 def _native_bias(source_counts, source_logit_biases, values):
     """(whether the native call can take the logit bias, the bias).  Raises nothing: what the Python
     checks would refuse, or pass over for a single source, is left to them."""
@@ -368,11 +371,11 @@ def _native_bias(source_counts, source_logit_biases, values):
     if not isinstance(values, (list, tuple)) or not isinstance(given, (list, tuple)):
         return False, None
     n = len(values)
-    if n < 2 or len(given) != n or not all(type(x) in (float, int) for x in given):
+    if n < 2 or len(given) != n or not _NUMBERS.issuperset(map(type, given)):
         return False, None
     if source_counts is not None and any(c <= 0 for c in given):
         return False, None
-    if not isinstance(values[0], Tensor) or not values[0].is_cuda:
+    if not getattr(values[0], "is_cuda", False):
         return False, None
     return True, _source_logit_bias(source_counts, source_logit_biases, n, values[0].device)
 
